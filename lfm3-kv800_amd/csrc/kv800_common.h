@@ -35,21 +35,11 @@ __device__ __forceinline__ float f8d(uint32_t b) {
 }
 
 // float -> fp8 e4m3fn byte with torch's .to(float8_e4m3fn) semantics (round to nearest even on the e4m3 grid,
-// results past 448 and inf / NaN -> 0x7F with the sign bit)
+// results past 448 and inf / NaN -> 0x7F with the sign bit). The hardware conversion does that for every float but NaN
+// (compared over all 2^32 against the bit arithmetic), whose sign it drops.
 __device__ __forceinline__ uint32_t f8e(float f) {
-  const uint32_t x = __float_as_uint(f);
-  const uint32_t sign = (x >> 24) & 0x80u;
-  const uint32_t a = x & 0x7FFFFFFFu;
-  if (a >= 0x7F800000u) return sign | 0x7Fu;
-  const float v = __uint_as_float(a);
-  if (v < 0.015625f) return sign | (uint32_t)__builtin_rintf(v * 512.0f);   // subnormal grid, step 2^-9
-  uint32_t keep = (a >> 20) & 7u, rest = a & 0xFFFFFu, e8 = ((a >> 23) & 0xFFu) - 120u;
-  if (rest > 0x80000u || (rest == 0x80000u && (keep & 1u))) {
-    keep += 1u;
-    if (keep == 8u) { keep = 0u; e8 += 1u; }
-  }
-  if (e8 > 15u || (e8 == 15u && keep == 7u)) return sign | 0x7Fu;
-  return sign | (e8 << 3) | keep;
+  const uint32_t r = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(f, f, 0, false) & 0xFFu;
+  return f == f ? r : ((__float_as_uint(f) >> 24) & 0x80u) | 0x7Fu;
 }
 
 __device__ __forceinline__ float clamp_min_1e8(float a) { return a < 1e-8f ? 1e-8f : a; }

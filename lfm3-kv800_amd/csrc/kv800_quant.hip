@@ -41,7 +41,8 @@ int check_launch(const char* what) {
 namespace {
 
 constexpr int QTHREADS = 512;    // 8 waves per sub-block, 32 tokens each
-constexpr int QW = QTHREADS / 64, TPW = BLK / QW;
+constexpr int QWPS = 4;          // waves per SIMD the throughput kernels are built for (two workgroups per CU)
+constexpr int QW = QTHREADS / 64;
 
 // ---------------------------------------------------------------- token-row sources
 struct DenseSrc {   // (M, 256, 4, 128) contiguous K and V
@@ -58,17 +59,23 @@ struct PagedSrc {   // exact pages: K of (position p, head h) at eoff[r, p / ebs
   const int64_t* et;   // this row's page table
   int64_t ebs, e_hs, e_ts, e_v, p0;
   const int64_t* rowoff = nullptr;   // LDS: element offset of token t's head-0 K row, t < 256
-  // One page-table lookup and division per token for the whole workgroup (every thread must call it).
+  // Element offset of token t's head-0 K row. The division is a 32-bit one (20 instructions against 150) unless the
+  // positions or the page size need more (a scalar branch).
+  __device__ __forceinline__ int64_t row(int t) const {
+    const int64_t p = p0 + t;
+    if (((p0 + BLK) | ebs) >> 32) return et[p / ebs] + (p % ebs) * e_ts;
+    const uint32_t pg = (uint32_t)p / (uint32_t)ebs;
+    return et[pg] + (int64_t)((uint32_t)p - pg * (uint32_t)ebs) * e_ts;
+  }
+  // K pass: one page-table lookup per token for the whole workgroup (every thread must call it). A V lane reads one
+  // row per group of tokens and looks it up itself, without the barrier.
   __device__ void prepare(int64_t* tab) {
-    for (int t = threadIdx.x; t < BLK; t += blockDim.x) {
-      const int64_t p = p0 + t;
-      tab[t] = et[p / ebs] + (p % ebs) * e_ts;
-    }
+    for (int t = threadIdx.x; t < BLK; t += blockDim.x) tab[t] = row(t);
     __syncthreads();
     rowoff = tab;
   }
   __device__ const uint16_t* krow(int t, int h) const { return ep + rowoff[t] + h * e_hs; }
-  __device__ const uint16_t* vrow(int t, int h) const { return krow(t, h) + e_v; }
+  __device__ const uint16_t* vrow(int t, int h) const { return ep + row(t) + h * e_hs + e_v; }
 };
 
 // K code clamp(rne(fl(d / den)), 0, 3) without the division. fl(q) > 1/2 <=> d > den / 2 (a float above den / 2 is
@@ -90,186 +97,131 @@ __device__ __forceinline__ uint32_t row_ror(uint32_t x, int n) {
                 : (uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, 0x128, 0xF, 0xF, false);
 }
 
-struct QuantLds {                  // K path: per-wave min / max partials, then per-column lo and divisor
-  float red_min[QW][512];
-  float red_max[QW][512];
-  float col_lo[512];
-  float col_den[512];
-};
-
-// K codes and scales of one sub-block, all 4 heads in one workgroup: per (head, channel) min / max over its 256
-// tokens (8 waves x 32 tokens). The latency flush uses it (one workgroup per sub-block's K); the throughput grids
-// take the per-head form below, which reads each row once.
-template <typename Src, int KG = 4>
-__device__ void quantize_k(const Src& src, uint8_t* __restrict__ out, char* lds) {
-  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-  QuantLds& S = *reinterpret_cast<QuantLds*>(lds);
-  float* red_min = &S.red_min[0][0];
-  float* red_max = &S.red_max[0][0];
-  float* col_lo = S.col_lo;
-  float* col_den = S.col_den;
-
-  // ---------------- K: wave w = tokens 32w .. 32w + 31, lane = columns 8 lane .. 8 lane + 7 (head lane / 16). The
-  // rows are read in groups of KG tokens, twice (min / max, then codes): the code pass walks the groups in reverse, so
-  // it starts with the rows read last, the ones most likely still in L2 while the rest of the grid streams through it.
-  // KG = 4 keeps the pass within the 64 VGPRs of the V pass it shares a grid with (8 waves per SIMD).
-  const int h = lane >> 4, c0 = 8 * (lane & 15);
-  float mn[8], mx[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) { mn[e] = INFINITY; mx[e] = -INFINITY; }
-#pragma unroll 1
-  for (int t0 = 0; t0 < TPW; t0 += KG) {
-    uint4 kx[KG];
-#pragma unroll
-    for (int tt = 0; tt < KG; ++tt) kx[tt] = *reinterpret_cast<const uint4*>(src.krow(TPW * w + t0 + tt, h) + c0);
-#pragma unroll
-    for (int tt = 0; tt < KG; ++tt) {
-      const uint32_t wd[4] = {kx[tt].x, kx[tt].y, kx[tt].z, kx[tt].w};
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float x = (e & 1) ? bf2f_hi(wd[e >> 1]) : bf2f_lo(wd[e >> 1]);
-        mn[e] = fminf(mn[e], x);
-        mx[e] = fmaxf(mx[e], x);
-      }
-    }
-  }
-  const int hc0 = h * 128 + c0;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) { red_min[w * 512 + hc0 + e] = mn[e]; red_max[w * 512 + hc0 + e] = mx[e]; }
-  __syncthreads();
-  if (tid < 512) {
-    float lo = red_min[tid], hi = red_max[tid];
-#pragma unroll
-    for (int ww = 1; ww < QW; ++ww) { lo = fminf(lo, red_min[ww * 512 + tid]); hi = fmaxf(hi, red_max[ww * 512 + tid]); }
-    const uint32_t lo8 = f8e(lo);
-    const uint32_t sc8 = f8e(clamp_min_1e8(__fdiv_rn(__fsub_rn(hi, lo), 3.0f)));
-    out[KLO_O + tid] = (uint8_t)lo8;
-    out[KSC_O + tid] = (uint8_t)sc8;
-    col_lo[tid] = f8d(lo8);
-    col_den[tid] = clamp_min_1e8(f8d(sc8));
-  }
-  __syncthreads();
-  {
-    float lof[8], den[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) { lof[e] = col_lo[hc0 + e]; den[e] = col_den[hc0 + e]; }
-    const int p = (lane & 15) >> 2, q = lane & 3;   // plane of these 8 channels, byte quarter 8q .. 8q + 7
-#pragma unroll 1
-    for (int t0 = TPW - KG; t0 >= 0; t0 -= KG) {
-      uint4 kx[KG];
-#pragma unroll
-      for (int tt = 0; tt < KG; ++tt) kx[tt] = *reinterpret_cast<const uint4*>(src.krow(TPW * w + t0 + tt, h) + c0);
-#pragma unroll
-      for (int tt = 0; tt < KG; ++tt) {
-        __builtin_amdgcn_sched_barrier(0);   // one token row at a time
-        const uint32_t wd[4] = {kx[tt].x, kx[tt].y, kx[tt].z, kx[tt].w};
-        uint32_t d0 = 0, d1 = 0;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float x = (e & 1) ? bf2f_hi(wd[e >> 1]) : bf2f_lo(wd[e >> 1]);
-          const uint32_t code = kcode(__fsub_rn(x, lof[e]), den[e]) << (2 * p);
-          if (e < 4) d0 |= code << (8 * e); else d1 |= code << (8 * (e - 4));
-        }
-        // the 4 planes of these bytes sit in the lanes 4, 8, 12 apart within the 16-lane row
-        d0 |= row_ror(d0, 4); d1 |= row_ror(d1, 4);
-        d0 |= row_ror(d0, 8); d1 |= row_ror(d1, 8);
-        if (p == 0) {
-          const int t = TPW * w + t0 + tt;
-          *reinterpret_cast<uint2*>(out + KC_O + (t * 4 + h) * 32 + 8 * q) = make_uint2(d0, d1);
-        }
-      }
-    }
-  }
+// bf16 pairs as ordered 16-bit keys: the bits of a non-negative value as they are, a negative one's magnitude bits
+// flipped, so that signed 16-bit compares order the values (-0 below +0) and one packed instruction takes two of them.
+// The map is its own inverse. NaN keys lie outside [KEY_NINF, KEY_INF].
+typedef short s2 __attribute__((ext_vector_type(2)));
+constexpr int KEY_INF = 0x7F80, KEY_NINF = -32641;
+__device__ __forceinline__ uint32_t as_u(s2 x) { return __builtin_bit_cast(uint32_t, x); }
+__device__ __forceinline__ s2 as_s2(uint32_t x) { return __builtin_bit_cast(s2, x); }
+__device__ __forceinline__ s2 bf_keys(uint32_t w) {
+  const s2 x = as_s2(w);
+  return as_s2(w ^ (as_u(x >> (short)15) & 0x7FFF7FFFu));
+}
+__device__ __forceinline__ float key_float(int k) {   // the value of one key
+  return bf2f((uint32_t)(uint16_t)(k ^ ((k >> 15) & 0x7FFF)));
+}
+// min / max over the lanes l, l ^ 16, l ^ 32, l ^ 48
+template <bool MAX>
+__device__ __forceinline__ s2 reduce4rows(s2 x) {
+  auto r = __builtin_amdgcn_permlane16_swap(as_u(x), as_u(x), false, false);
+  x = MAX ? __builtin_elementwise_max(as_s2(r[0]), as_s2(r[1])) : __builtin_elementwise_min(as_s2(r[0]), as_s2(r[1]));
+  r = __builtin_amdgcn_permlane32_swap(as_u(x), as_u(x), false, false);
+  return MAX ? __builtin_elementwise_max(as_s2(r[0]), as_s2(r[1])) : __builtin_elementwise_min(as_s2(r[0]), as_s2(r[1]));
 }
 
 // K codes and scales of one head hh of one sub-block, its 256 token rows read once: lane (g, c) of wave w holds the
-// 8 channels 8 c .. 8 c + 7 of the tokens 32 i + 4 w + g (i = 0..7) in registers through both passes (min / max, then
-// codes), so each row is fetched from memory once (the all-heads pass above reads its rows twice). Min / max across
-// the 4 token rows of a wave by permlane swaps, across the 8 waves through LDS.
-struct QuantLds1 {
-  float red_min[QW][128];
-  float red_max[QW][128];
-  float col_lo[128];
-  float col_den[128];
+// 8 channels 8 c .. 8 c + 7 of the tokens 32 i + 4 w + g (i = 0..7) as key pairs in registers through both passes (min /
+// max, then codes). Min / max across the 4 token rows of a wave by permlane swaps, across the 8 waves through LDS.
+// d = fl(x - lo) never decreases with x and the code never with d, so a channel's code is the number of its three
+// thresholds T_c (the smallest bf16 value of code >= c) that x reaches: thread 128 c + channel computes T_c and settles
+// it with kcode itself. An element then costs 2 VALU instructions for min / max and 4 for its code, against 24 with the
+// arithmetic per element, and they matter because the V workgroups' fp32 MFMA and VALU share the part's FMA units.
+// A workgroup that holds a NaN takes the arithmetic per element (min / max skip NaN, its code is 0).
+struct QuantLds {
+  s2 red_min[QW][64], red_max[QW][64];   // per wave, channel pairs
+  short thr[3][128];                     // T_c - 1
+  float lo[128], den[128];
 };
-__device__ __forceinline__ float min4rows(float x) {
-  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  x = fminf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-  r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return fminf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-__device__ __forceinline__ float max4rows(float x) {
-  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  x = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-  r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
 template <typename Src>
-__device__ void quantize_k1(const Src& src, uint8_t* __restrict__ out, char* lds, int hh) {
+__device__ void quantize_k(const Src& src, uint8_t* __restrict__ out, char* lds, int hh) {
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, g = lane >> 4, c16 = lane & 15, c0 = 8 * c16;
-  QuantLds1& S = *reinterpret_cast<QuantLds1*>(lds);
+  QuantLds& S = *reinterpret_cast<QuantLds*>(lds);
   constexpr int NT = BLK / 32;   // tokens per lane
-  uint4 kx[NT];
-#pragma unroll
-  for (int i = 0; i < NT; ++i) kx[i] = *reinterpret_cast<const uint4*>(src.krow(32 * i + 4 * w + g, hh) + c0);
+  s2 kx[NT][4];
   {
-    float mn[8], mx[8];
+    uint4 raw[NT];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) { mn[e] = INFINITY; mx[e] = -INFINITY; }
+    for (int i = 0; i < NT; ++i) raw[i] = *reinterpret_cast<const uint4*>(src.krow(32 * i + 4 * w + g, hh) + c0);
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
-      __builtin_amdgcn_sched_barrier(0);   // one token row at a time
-      const uint32_t wd[4] = {kx[i].x, kx[i].y, kx[i].z, kx[i].w};
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float x = (e & 1) ? bf2f_hi(wd[e >> 1]) : bf2f_lo(wd[e >> 1]);
-        mn[e] = fminf(mn[e], x);
-        mx[e] = fmaxf(mx[e], x);
-      }
-    }
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      __builtin_amdgcn_sched_barrier(0);
-      mn[e] = min4rows(mn[e]);
-      mx[e] = max4rows(mx[e]);
-    }
-    if (g == 0) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) { S.red_min[w][c0 + e] = mn[e]; S.red_max[w][c0 + e] = mx[e]; }
+      kx[i][0] = bf_keys(raw[i].x); kx[i][1] = bf_keys(raw[i].y);
+      kx[i][2] = bf_keys(raw[i].z); kx[i][3] = bf_keys(raw[i].w);
     }
   }
-  __syncthreads();
-  if (tid < 128) {
-    float lo = S.red_min[0][tid], hi = S.red_max[0][tid];
+  bool nan = false;
 #pragma unroll
-    for (int ww = 1; ww < QW; ++ww) { lo = fminf(lo, S.red_min[ww][tid]); hi = fmaxf(hi, S.red_max[ww][tid]); }
+  for (int d = 0; d < 4; ++d) {
+    s2 mn = kx[0][d], mx = kx[0][d];
+#pragma unroll
+    for (int i = 1; i < NT; ++i) {
+      mn = __builtin_elementwise_min(mn, kx[i][d]);
+      mx = __builtin_elementwise_max(mx, kx[i][d]);
+    }
+    mn = reduce4rows<false>(mn);
+    mx = reduce4rows<true>(mx);
+    nan |= mn.x < KEY_NINF || mn.y < KEY_NINF || mx.x > KEY_INF || mx.y > KEY_INF;
+    if (g == 0) { S.red_min[w][4 * c16 + d] = mn; S.red_max[w][4 * c16 + d] = mx; }
+  }
+  nan = __syncthreads_or(nan);   // uniform over the workgroup
+  if (nan) {                     // min / max of the values that are no NaN (none: +inf, -inf), as fminf / fmaxf give
+    __syncthreads();
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      s2 mn = {(short)KEY_INF, (short)KEY_INF}, mx = {(short)KEY_NINF, (short)KEY_NINF};
+#pragma unroll
+      for (int i = 0; i < NT; ++i) {
+        const s2 k = kx[i][d];
+        if (k.x >= KEY_NINF && k.x <= KEY_INF) { mn.x = min(mn.x, k.x); mx.x = max(mx.x, k.x); }
+        if (k.y >= KEY_NINF && k.y <= KEY_INF) { mn.y = min(mn.y, k.y); mx.y = max(mx.y, k.y); }
+      }
+      mn = reduce4rows<false>(mn);
+      mx = reduce4rows<true>(mx);
+      if (g == 0) { S.red_min[w][4 * c16 + d] = mn; S.red_max[w][4 * c16 + d] = mx; }
+    }
+    __syncthreads();
+  }
+  {
+    const int col = tid & 127, c = tid >> 7;
+    int kmn = reinterpret_cast<const short*>(S.red_min[0])[col], kmx = reinterpret_cast<const short*>(S.red_max[0])[col];
+#pragma unroll
+    for (int ww = 1; ww < QW; ++ww) {
+      kmn = min(kmn, (int)reinterpret_cast<const short*>(S.red_min[ww])[col]);
+      kmx = max(kmx, (int)reinterpret_cast<const short*>(S.red_max[ww])[col]);
+    }
+    const float lo = key_float(kmn), hi = key_float(kmx);
     const uint32_t lo8 = f8e(lo);
     const uint32_t sc8 = f8e(clamp_min_1e8(__fdiv_rn(__fsub_rn(hi, lo), 3.0f)));
-    out[KLO_O + hh * 128 + tid] = (uint8_t)lo8;
-    out[KSC_O + hh * 128 + tid] = (uint8_t)sc8;
-    S.col_lo[tid] = f8d(lo8);
-    S.col_den[tid] = clamp_min_1e8(f8d(sc8));
+    const float lof = f8d(lo8), den = clamp_min_1e8(f8d(sc8));
+    if (c == 0) {   // uniform over the wave
+      out[KLO_O + hh * 128 + col] = (uint8_t)lo8;
+      out[KSC_O + hh * 128 + col] = (uint8_t)sc8;
+      S.lo[col] = lof;
+      S.den[col] = den;
+    } else {
+      auto reaches = [&](int k) { return kcode(__fsub_rn(key_float(k), lof), den) >= (uint32_t)c; };
+      // D: the smallest d of code >= c (an ulp or two about (c - 1/2) den, which is exact); then x with x - lo at the
+      // rounding midpoint below D, exact or to an fp32 rounding of x itself
+      const uint32_t base = __float_as_uint(((float)c - 0.5f) * den);
+      uint32_t db = base - 1;
+#pragma unroll
+      for (int k = -1; k < 2; ++k) db += kcode(__uint_as_float(base + k), den) < (uint32_t)c;
+      const float D = __uint_as_float(db);
+      const float x0 = __fsub_rn(__fadd_rn(lof, D), 0.5f * __fsub_rn(D, __uint_as_float(db - 1)));
+      const int k0 = as_s2(as_u(bf_keys(f2bf(x0)))).x;
+      int a = k0 - 1, b = k0 + 1;   // T_c in (a, b], or anywhere when either end says otherwise
+      if (reaches(a)) a = KEY_NINF - 1;
+      if (!reaches(b)) b = KEY_INF + 1;
+      while (b - a > 1) {
+        const int mid = (a + b) >> 1;
+        if (reaches(mid)) b = mid; else a = mid;
+      }
+      S.thr[c - 1][col] = (short)(b - 1);
+    }
   }
   __syncthreads();
-  // the rows stay packed across the passes: their unpacked floats are formed again here, not kept from the first
-  // pass (64 registers instead of 32)
-#pragma unroll
-  for (int i = 0; i < NT; ++i) asm volatile("" : "+v"(kx[i].x), "+v"(kx[i].y), "+v"(kx[i].z), "+v"(kx[i].w));
-  float lof[8], den[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) { lof[e] = S.col_lo[c0 + e]; den[e] = S.col_den[c0 + e]; }
   const int p = c16 >> 2, q = c16 & 3;   // plane of these 8 channels, byte quarter 8q .. 8q + 7
-#pragma unroll
-  for (int i = 0; i < NT; ++i) {
-    __builtin_amdgcn_sched_barrier(0);   // one token row at a time
-    const uint32_t wd[4] = {kx[i].x, kx[i].y, kx[i].z, kx[i].w};
-    uint32_t d0 = 0, d1 = 0;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float x = (e & 1) ? bf2f_hi(wd[e >> 1]) : bf2f_lo(wd[e >> 1]);
-      const uint32_t code = kcode(__fsub_rn(x, lof[e]), den[e]) << (2 * p);
-      if (e < 4) d0 |= code << (8 * e); else d1 |= code << (8 * (e - 4));
-    }
+  auto store = [&](int i, uint32_t d0, uint32_t d1) {
     // the 4 planes of these bytes sit in the lanes 4, 8, 12 apart within the 16-lane row
     d0 |= row_ror(d0, 4); d1 |= row_ror(d1, 4);
     d0 |= row_ror(d0, 8); d1 |= row_ror(d1, 8);
@@ -277,6 +229,50 @@ __device__ void quantize_k1(const Src& src, uint8_t* __restrict__ out, char* lds
       const int t = 32 * i + 4 * w + g;
       *reinterpret_cast<uint2*>(out + KC_O + (t * 4 + hh) * 32 + 8 * q) = make_uint2(d0, d1);
     }
+  };
+  if (nan) {
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      __builtin_amdgcn_sched_barrier(0);
+      uint32_t dw[2] = {0, 0};
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int k = (e & 1) ? kx[i][e >> 1].y : kx[i][e >> 1].x;
+        dw[e >> 2] |= kcode(__fsub_rn(key_float(k), S.lo[c0 + e]), S.den[c0 + e]) << (2 * p + 8 * (e & 3));
+      }
+      store(i, dw[0], dw[1]);
+    }
+    return;
+  }
+  s2 th[3][4];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    const uint4 t = *reinterpret_cast<const uint4*>(&S.thr[c][c0]);
+    th[c][0] = as_s2(t.x); th[c][1] = as_s2(t.y); th[c][2] = as_s2(t.z); th[c][3] = as_s2(t.w);
+  }
+#pragma unroll
+  for (int i = 0; i < NT; ++i) {
+    __builtin_amdgcn_sched_barrier(0);   // one token row at a time
+    // sign bits: u_c = x >= T_c; the code's high bit is u_2, its low bit u_3 where u_2, else u_1
+    uint32_t dw[2];
+#pragma unroll
+    for (int d = 0; d < 2; ++d) {
+      uint32_t lb[2], hb[2];
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const s2 x = kx[i][2 * d + k];
+        const uint32_t u1 = as_u(__builtin_elementwise_sub_sat(th[0][2 * d + k], x));
+        const uint32_t u2 = as_u(__builtin_elementwise_sub_sat(th[1][2 * d + k], x));
+        const uint32_t u3 = as_u(__builtin_elementwise_sub_sat(th[2][2 * d + k], x));
+        lb[k] = (u2 & u3) | (~u2 & u1);
+        hb[k] = u2;
+      }
+      // the 4 channels' sign bytes side by side, then code bits 7 and 6 of each byte down to the plane's two bits
+      const uint32_t lw = __builtin_amdgcn_perm(lb[1], lb[0], 0x07050301u);
+      const uint32_t hw = __builtin_amdgcn_perm(hb[1], hb[0], 0x07050301u);
+      dw[d] = (((hw & 0x80808080u) | ((lw >> 1) & 0x7F7F7F7Fu)) & 0xC0C0C0C0u) >> (6 - 2 * p);
+    }
+    store(i, dw[0], dw[1]);
   }
 }
 
@@ -377,105 +373,324 @@ __device__ __forceinline__ VScales v_scales(const float (&y)[8], int lane) {
   return VScales{b8, g ? lof1 : lof0, scf, clamp_min_1e8(scf)};
 }
 
-// V bits and scales of tokens [t0, t0 + VT * QW) of one sub-block: wave w takes VT consecutive tokens, one token (its
-// 4 head rows) per step. Each lane loads 16 bytes of the token's rows (head hh, dims 8 jj .. 8 jj + 7), two tokens
-// ahead; the wave writes them as floats into its own LDS rows, and each lane runs its row's 8-output chain from there.
-// Per (token, 2-head group) -- lanes 32 g .. 32 g + 31 -- the min / max of the 256 outputs go through a 16-row swap and
-// DPP row reductions; the token's four scale bytes (lo and scale of each group) are encoded by lanes 0..3 at once.
-// bit = rne(fl(d / den)) >= 1 with d = fl(y - lo) is evaluated without the division as d > den / 2: a float d above
-// den / 2 exceeds it by at least an ulp of den / 2, so d / den > 1/2 + 2^-25 and the quotient rounds above 1/2; at
-// d = den / 2 it is 1/2, which rounds to 0 (den >= 1e-8 is normal; a NaN den or d gives 0 both ways).
-constexpr int VSPLIT = 4, VTOK = BLK / VSPLIT, VTPW = VTOK / QW;
-constexpr int VROW = 132;   // floats per staged row: the 4 rows of a token start on different LDS banks
-constexpr int VLDS_BYTES = QW * 4 * VROW * 4;
-
-template <int VT, typename Src>
-__device__ void quantize_v(const Src& src, uint8_t* __restrict__ out, int t0, char* lds) {
-  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-  const int tw = t0 + VT * w;                    // this wave's first token
-  const int hh = lane >> 4, jj = lane & 15;      // head row and code byte of this lane
-  float* xrow = reinterpret_cast<float*>(lds) + (w * 4 + hh) * VROW;
-  auto fetch = [&](int t) { return *reinterpret_cast<const uint4*>(src.vrow(t, hh) + 8 * jj); };
-  uint4 pf0 = fetch(tw), pf1 = VT > 1 ? fetch(tw + 1) : pf0;
-  float hl[16];
-  hadamard_low(hl, jj);
-  const int q = lane & 3;
-#pragma unroll 1
-  for (int tt = 0; tt < VT; ++tt) {
-    const int t = tw + tt;
-    // token t's rows -> LDS (a wave's LDS instructions execute in order: these stores follow the previous token's
-    // reads and precede this token's)
-    float4* dst = reinterpret_cast<float4*>(xrow + 8 * jj);
-    dst[0] = make_float4(bf2f_lo(pf0.x), bf2f_hi(pf0.x), bf2f_lo(pf0.y), bf2f_hi(pf0.y));
-    dst[1] = make_float4(bf2f_lo(pf0.z), bf2f_hi(pf0.z), bf2f_lo(pf0.w), bf2f_hi(pf0.w));
-    pf0 = pf1;
-    if (tt + 2 < VT) pf1 = fetch(t + 2);
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    float y[8];
-    hadamard_row8(xrow, hl, y);
-
-    const VScales sc = v_scales(y, lane);
-    if (lane < 4) out[((q & 1) ? VSC_O : VLO_O) + t * 2 + (q >> 1)] = (uint8_t)sc.b8;
-    const float half = sc.den * 0.5f;
-    uint32_t byte = 0;
+// ---------------------------------------------------------------- V path on the fp32 matrix cores
+// y = x H for 16 head rows at once (4 tokens x 4 heads; row m = 4 token + head), every output still the sequential fma
+// chain over k = 0..127: v_mfma_f32_16x16x4_f32 adds its four products to the accumulator one after another, k
+// ascending, each as one IEEE fma (denormals, infinities and NaN included; measured against the scalar chain bit for
+// bit), so 32 steps of four k make the chain. Prefixes are shared as in hadamard_row8: tile i holds dims j + 16 i
+// (column j), one tile for k < 16, two for k < 32, four for k < 64, eight after: 172 MFMA for 16 rows' 2,048 outputs.
+// Why: the part issues 75 T fp32 fma/s through MFMA and sustained 35 T through these vector chains.
+//   A operand: lane (g, m) = (lane / 16, lane % 16) holds x[m][4 s + g] in x[s];
+//   B operand: H[4 s + g][j] for s < 4 (the other k differ by hneg's sign), and its negation;
+//   result:    lane (g, j), y[i][r] = output j + 16 i of row 4 g + r: the lane's eight tiles at one r are the eight
+//              bits of code byte j of head r of token g.
+typedef float f4 __attribute__((ext_vector_type(4)));
+struct HadB { f4 p, n; };   // element s & 3
+__device__ __forceinline__ HadB had_operand(int lane) {
+  const float c = __uint_as_float(0x3DB504F3u);   // fp32(1 / sqrt(128))
+  auto h = [&](int s) { return (__popc((4 * s + (lane >> 4)) & (lane & 15)) & 1) ? -c : c; };
+  const f4 p = {h(0), h(1), h(2), h(3)};
+  return HadB{p, -p};
+}
+// conv(in[q], x) delivers x[m][4 s + g], s = 8 q .. 8 q + 7, as the chain reaches them
+template <typename T, typename Conv>
+__device__ __forceinline__ void hadamard_rows16(const T (&in)[4], Conv conv, const HadB& b, f4 (&y)[8]) {
+  y[0] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int i = 0; i < 8; ++i) byte |= (__fsub_rn(y[i], sc.lof) > half) ? (1u << i) : 0u;
-    out[VB_O + t * 64 + lane] = (uint8_t)byte;
+  for (int q = 0; q < 4; ++q) {
+    float x[8];
+    conv(in[q], x);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int s = 8 * q + u, m = s >> 2, nch = m == 0 ? 1 : m == 1 ? 2 : m < 4 ? 4 : 8;
+      if (s == 4 || s == 8 || s == 16) {
+#pragma unroll
+        for (int i = 0; i < nch / 2; ++i) y[nch / 2 + i] = y[i];
+      }
+#pragma unroll
+      for (int i = 0; i < nch; ++i)
+        y[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[u], hneg(m, i) ? b.n[s & 3] : b.p[s & 3], y[i], 0, 0, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);   // one piece's x at a time
   }
 }
 
-// A quantize grid holds, per sub-block, 4 K workgroups (one per head: all 256 tokens per channel, each row read once)
-// followed in the grid by VSPLIT V workgroups (V is independent per token). Both passes fit 72 VGPRs and 39 KB of LDS,
-// so 7 waves per SIMD run and the K workgroups' memory latency overlaps the V workgroups' fma chains. Workgroup
-// i < 4 units is the K pass of unit i / 4, head i % 4; i >= 4 units is the V pass of unit (i - 4 units) / VSPLIT, token
-// range (i - 4 units) % VSPLIT.
-constexpr int QLDS_BYTES = (int)sizeof(QuantLds) > VLDS_BYTES ? (int)sizeof(QuantLds) : VLDS_BYTES;
-static_assert(sizeof(QuantLds1) <= (size_t)QLDS_BYTES, "per-head K pass LDS");
+// 4 x 4 transpose between four registers and the lanes l, l ^ 16, l ^ 32, l ^ 48: lane group g's register e becomes
+// register g of lane group e. All 64 lanes must be active.
+__device__ __forceinline__ void transpose_rows4(float& a0, float& a1, float& a2, float& a3) {
+  auto sw32 = [](float& u, float& v) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(u), __float_as_uint(v), false, false);
+    u = __uint_as_float(r[0]); v = __uint_as_float(r[1]);
+  };
+  auto sw16 = [](float& u, float& v) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(u), __float_as_uint(v), false, false);
+    u = __uint_as_float(r[0]); v = __uint_as_float(r[1]);
+  };
+  sw32(a0, a2); sw32(a1, a3);
+  sw16(a0, a1); sw16(a2, a3);
+}
+
+// x of lane's dpp partner inside its quad (CTRL: a quad_perm control word)
+template <int CTRL>
+__device__ __forceinline__ uint32_t quad(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, CTRL, 0xF, 0xF, false);
+}
+template <int CTRL>
+__device__ __forceinline__ float quadf(float x) { return __uint_as_float(quad<CTRL>(__float_as_uint(x))); }
+constexpr int QUAD0 = 0x00, QUAD1 = 0x55, QUAD2 = 0xAA, QUAD3 = 0xFF, QUAD_X1 = 0xB1, QUAD_X2 = 0x4E;
+
+// Scales of four tokens' V rows from y (lane (g, j): token g): per 2-head pair (r = 0, 1 and r = 2, 3) the min and max
+// of its 256 outputs, in-lane, then over the token's 16 lanes by DPP row reductions; lane j encodes byte q = j & 3 of
+// its token: lo (q even) or max(hi - lo, 1e-8) (q odd) of pair q >> 1. lof / scf: both pairs' decoded lo and scale.
+struct VScales4 { uint32_t b8; float lof[2], scf[2]; };
+__device__ __forceinline__ VScales4 v_scales4(const f4 (&y)[8], int lane) {
+  const int q = lane & 3;
+  float lo[2], hi[2];
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    float mn = fminf(y[0][2 * p], y[0][2 * p + 1]), mx = fmaxf(y[0][2 * p], y[0][2 * p + 1]);
+#pragma unroll
+    for (int i = 1; i < 8; ++i) {
+      mn = fminf(fminf(mn, y[i][2 * p]), y[i][2 * p + 1]);
+      mx = fmaxf(fmaxf(mx, y[i][2 * p]), y[i][2 * p + 1]);
+    }
+    lo[p] = row_min16(mn);
+    hi[p] = -row_min16(-mx);
+  }
+  const float glo = (q & 2) ? lo[1] : lo[0], ghi = (q & 2) ? hi[1] : hi[0];
+  VScales4 s;
+  s.b8 = f8e((q & 1) ? clamp_min_1e8(__fsub_rn(ghi, glo)) : glo);
+  const float dec = f8d(s.b8);
+  s.lof[0] = quadf<QUAD0>(dec); s.scf[0] = quadf<QUAD1>(dec);
+  s.lof[1] = quadf<QUAD2>(dec); s.scf[1] = quadf<QUAD3>(dec);
+  return s;
+}
+
+// Code bytes of four tokens' V rows, packed: byte r of the result is byte j of head r of token g. bit = rne(fl(d / den))
+// >= 1 with d = fl(y - lo) is evaluated without the division as d > den / 2: a float d above den / 2 exceeds it by at
+// least an ulp of den / 2, so d / den > 1/2 + 2^-25 and the quotient rounds above 1/2; at d = den / 2 it is 1/2, which
+// rounds to 0 (den >= 1e-8 is normal; a NaN den or d gives 0 both ways).
+__device__ __forceinline__ uint32_t v_bits4(const f4 (&y)[8], const VScales4& s) {
+  uint32_t w = 0;
+#pragma unroll
+  for (int r = 3; r >= 0; --r) {
+    const float lo = s.lof[r >> 1], half = clamp_min_1e8(s.scf[r >> 1]) * 0.5f;
+#pragma unroll
+    for (int i = 7; i >= 0; --i) {   // w = 2 w + bit, the compare's mask as the carry
+      const float d = __fsub_rn(y[i][r], lo);
+      asm("v_cmp_gt_f32 vcc, %1, %2\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(w) : "v"(d), "v"(half) : "vcc");
+    }
+  }
+  return w;
+}
+// 4 x 4 byte transpose within each quad of lanes: byte r of lane e becomes byte e of lane r, so that lane j = 4 a + e
+// holds bytes 4 a .. 4 a + 3 of head e.
+__device__ __forceinline__ uint32_t quad_bytes(uint32_t w, int lane) {
+  const uint32_t x = quad<QUAD_X1>(w);
+  const uint32_t v = __builtin_amdgcn_perm(w, x, (lane & 1) ? 0x07030501u : 0x02060004u);
+  const uint32_t z = quad<QUAD_X2>(v);
+  return __builtin_amdgcn_perm(v, z, (lane & 2) ? 0x07060302u : 0x01000504u);
+}
+
+// The quantizer needs the chain's value only where rounding decides a byte. Its fast form takes y' = c D, D = sum of
+// the +-x by v_mfma_f32_16x16x32_bf16 (x and +-1 are exact in bf16; 36 MFMA at twice the rate per instruction and off
+// the VALU, which the fp32 MFMA occupies), with a bound on |y' - y|: the chain rounds 128 times, each time by at most
+// 2^-24 of a partial sum that is at most c l1, l1 = sum |x| of the row, and D is within 9 2^-24 l1 of the exact sum (the
+// largest deviation measured on cancelling, wide-range and denormal rows; 32 is allowed), so |D - y / c| <= 160 2^-24 l1.
+// With E = 192 2^-24 l1 (and 1e-30 for flushed denormals) a group of four tokens is done if for every scale byte both
+// ends of the value's interval encode alike and every D keeps E plus the threshold's own rounding from its bit's
+// threshold; otherwise (one group in six for normal values; infinities and NaN always) the exact chain runs. All
+// bytes are those of the chain. Per group of four tokens: 7.1 K cycles of a SIMD for the exact chain alone, about 2.5 K
+// for this form with its share of exact ones.
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u4v __attribute__((ext_vector_type(4)));
+struct SignB { u4v even, odd; };   // B operand k = 32 q + 8 g + e, column j + 16 i: set i & 1, negated by parity(q & i >> 1)
+__device__ __forceinline__ SignB sign_operand(int lane) {
+  const int g = lane >> 4, j = lane & 15;
+  auto pair = [&](int d) {
+    return 0x3F803F80u | ((uint32_t)(__popc((8 * g + 2 * d) & j) & 1) << 15) |
+           ((uint32_t)(__popc((8 * g + 2 * d + 1) & j) & 1) << 31);
+  };
+  SignB b;
+  b.even = u4v{pair(0), pair(1), pair(2), pair(3)};
+  b.odd = b.even ^ ((g & 2) ? 0x80008000u : 0u);
+  return b;
+}
+__device__ __forceinline__ f4 mfma_bf(u4v a, u4v b, f4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8, a), __builtin_bit_cast(b8, b), c, 0, 0, 0);
+}
+constexpr float VE_L1 = 192.f * 0x1p-24f, VE_ABS = 1e-30f, HC = 0x1.6a09e6p-4f, HC_INV = 0x1.6a09e6p+3f;
+
+// The fast form on one group's raw rows: in[q] = dims 32 q + 8 g .. + 7 of row m in lane (g, m). True where every byte
+// is settled (the same in all lanes); b8 is then lane j's scale byte, w the packed code bytes as v_bits4 gives them.
+__device__ __forceinline__ bool quick_v4(const uint4 (&in)[4], const SignB& sb, int lane, uint32_t& b8, uint32_t& w) {
+  f4 D[8], N = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < 8; ++i) D[i] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const u4v a = {in[q].x, in[q].y, in[q].z, in[q].w};
+    const u4v one = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
+    const u4v na = a ^ 0x80008000u;
+    N = mfma_bf(a & 0x7FFF7FFFu, one, N);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      D[i] = mfma_bf((__builtin_popcount(q & (i >> 1)) & 1) ? na : a, (i & 1) ? sb.odd : sb.even, D[i]);
+  }
+  const int q = lane & 3;
+  float lo[2], hi[2];
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    float mn = fminf(D[0][2 * p], D[0][2 * p + 1]), mx = fmaxf(D[0][2 * p], D[0][2 * p + 1]);
+#pragma unroll
+    for (int i = 1; i < 8; ++i) {
+      mn = fminf(fminf(mn, D[i][2 * p]), D[i][2 * p + 1]);
+      mx = fmaxf(fmaxf(mx, D[i][2 * p]), D[i][2 * p + 1]);
+    }
+    lo[p] = row_min16(mn);
+    hi[p] = -row_min16(-mx);
+  }
+  float E[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) E[r] = N[r] * VE_L1 + VE_ABS;
+  const float e2 = (q & 2) ? fmaxf(E[2], E[3]) : fmaxf(E[0], E[1]);
+  const float glo = (q & 2) ? lo[1] : lo[0], ghi = (q & 2) ? hi[1] : hi[0];
+  const float mid = ((q & 1) ? ghi - glo : glo) * HC, rad = e2 * ((q & 1) ? 2.f * HC : HC);
+  float va = mid - rad, vb = mid + rad;
+  if (q & 1) { va = clamp_min_1e8(va); vb = clamp_min_1e8(vb); }
+  // the hardware conversion gives f8e's byte for every finite float (checked over all of them)
+  const uint32_t ends = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(va, vb, 0, false);
+  b8 = ends & 0xFFu;
+  bool ok = b8 == ((ends >> 8) & 0xFFu);
+  const float dec = f8d(b8);
+  const float lof[2] = {quadf<QUAD0>(dec), quadf<QUAD2>(dec)}, scf[2] = {quadf<QUAD1>(dec), quadf<QUAD3>(dec)};
+  float T[2], slack[2];
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {   // bit: D > T, T = (lo + den / 2) / c
+    const float half = clamp_min_1e8(scf[p]) * 0.5f;
+    T[p] = (lof[p] + half) * HC_INV;
+    slack[p] = (fabsf(lof[p]) + half) * (HC_INV * 0x1p-20f);
+  }
+  w = 0;
+#pragma unroll
+  for (int r = 3; r >= 0; --r) {
+    float least = INFINITY;
+#pragma unroll
+    for (int i = 7; i >= 0; --i) {
+      const float t = D[i][r] - T[r >> 1];
+      least = fminf(least, fabsf(t));
+      asm("v_cmp_lt_f32 vcc, 0, %1\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(w) : "v"(t) : "vcc");
+    }
+    ok = ok && least > E[r] + slack[r >> 1];   // false for NaN and infinite l1
+  }
+  return __all(ok);
+}
+
+// V bits and scales of tokens [t0, t0 + 4 VG QW) of one sub-block: wave w takes VG groups of four consecutive tokens.
+// Lane (g, m) loads dims 8 g + 32 q .. + 7 of row m (four 16-byte pieces, every group's requested up front), the bf16 MFMA's A operand as
+// they are; for the exact chain the pieces' elements change places with the other lane groups' so
+// that the lane holds x[m][4 s + g].
+constexpr int VSPLIT = 4, VTOK = BLK / VSPLIT, VTPW = VTOK / QW;
+constexpr int VROW = 132;   // floats per staged row: the 4 rows of a token start on different LDS banks
+
+// Elements 4 u + e (u < 2, e < 4) of the 16-byte bf16 pieces 8 g' + 32 q in the lane groups g' -> lane group g's
+// x[2 g' + u] = element 4 u + g of group g', i.e. k = 4 (8 q + 2 g' + u) + g
+__device__ __forceinline__ void unpack_piece(const uint4& in, float (&x)[8]) {
+  float f[8] = {bf2f_lo(in.x), bf2f_hi(in.x), bf2f_lo(in.y), bf2f_hi(in.y),
+                bf2f_lo(in.z), bf2f_hi(in.z), bf2f_lo(in.w), bf2f_hi(in.w)};
+  transpose_rows4(f[0], f[1], f[2], f[3]);
+  transpose_rows4(f[4], f[5], f[6], f[7]);
+#pragma unroll
+  for (int gg = 0; gg < 4; ++gg) { x[2 * gg] = f[gg]; x[2 * gg + 1] = f[4 + gg]; }
+}
+
+template <int VG, typename Src>
+__device__ void quantize_v(const Src& src, uint8_t* __restrict__ out, int t0) {
+  const int lane = threadIdx.x & 63, g = lane >> 4, m = lane & 15;
+  const int tw = t0 + 4 * VG * (threadIdx.x >> 6);   // this wave's first token
+  uint4 raw[VG][4];
+#pragma unroll
+  for (int v = 0; v < VG; ++v) {
+    const uint16_t* row = src.vrow(tw + 4 * v + (m >> 2), m & 3) + 8 * g;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) raw[v][q] = *reinterpret_cast<const uint4*>(row + 32 * q);
+  }
+  const SignB sb = sign_operand(lane);
+#pragma unroll
+  for (int v = 0; v < VG; ++v) {
+    const uint4 (&in)[4] = raw[v];
+    uint32_t b8, w;
+    if (!quick_v4(in, sb, lane, b8, w)) {   // uniform over the wave
+      f4 y[8];
+      hadamard_rows16(in, unpack_piece, had_operand(lane), y);
+      const VScales4 sc = v_scales4(y, lane);
+      b8 = sc.b8;
+      w = v_bits4(y, sc);
+    }
+    const int t = tw + 4 * v + g;
+    if (m < 4) out[((m & 1) ? VSC_O : VLO_O) + t * 2 + (m >> 1)] = (uint8_t)b8;
+    *reinterpret_cast<uint32_t*>(out + VB_O + t * 64 + (m & 3) * 16 + (m & ~3)) = quad_bytes(w, lane);
+  }
+}
+
+// A quantize grid holds, per sub-block, VSPLIT V workgroups (V is independent per token) and 4 K workgroups (one per
+// head: all 256 tokens per channel, each row read once). All V workgroups come first: they are the long ones, and the K
+// workgroups fill in behind them (448 sub-blocks: 91 us, 98-118 us interleaved, 100 us with K first). V alone takes
+// 65 us, K alone 40 us, both mostly the latency of one-shot workgroups at two per CU; 448 sub-blocks of paged rows took
+// 147 us with a scalar fma chain per V lane and the code arithmetic per K element, and take 90 us now (2.9 TB/s).
+// 32-bit throughout (the host bounds the grid): scalar compares and selects.
+struct Part { int unit; bool kpass; int part; };
+__device__ __forceinline__ Part part_of(int units, int vsplit) {
+  const int i = (int)blockIdx.x;
+  const int nv = vsplit * units;
+  const bool k = i >= nv;
+  const int o = k ? i - nv : i, n = k ? 4 : vsplit;
+  return Part{o / n, k, o % n};
+}
 
 // kpass: part = the head of the per-head K pass; else the V token range
 template <typename Src>
-__device__ __forceinline__ void quantize_part(const Src& src, uint8_t* __restrict__ out, char* lds, bool kpass, int part) {
-  if (kpass) quantize_k1(src, out, lds, part);
-  else quantize_v<VTPW>(src, out, part * VTOK, lds);
+__device__ __forceinline__ void quantize_part(Src& src, uint8_t* __restrict__ out, char* lds, int64_t* rowtab, bool kpass,
+                                              int part) {
+  if (kpass) {
+    src.prepare(rowtab);
+    quantize_k(src, out, lds, part);
+  }
+  else quantize_v<VTPW / 4>(src, out, part * VTOK);
 }
 
-__global__ void __launch_bounds__(QTHREADS) quantize_dense_kernel(const uint16_t* __restrict__ k,
+__global__ void __launch_bounds__(QTHREADS, QWPS) quantize_dense_kernel(const uint16_t* __restrict__ k,
                                                                    const uint16_t* __restrict__ v,
                                                                    uint8_t* __restrict__ out, int64_t M) {
-  __shared__ __align__(16) char lds[QLDS_BYTES];
-  const int64_t i = blockIdx.x;
-  const bool kpass = i < 4 * M;
-  const int64_t m = kpass ? i / 4 : (i - 4 * M) / VSPLIT;
-  quantize_part(DenseSrc{k, v, m}, out + m * SUB, lds, kpass, kpass ? (int)(i % 4) : (int)((i - 4 * M) % VSPLIT));
+  __shared__ __align__(16) char lds[sizeof(QuantLds)];
+  const Part p = part_of((int)M, VSPLIT);
+  DenseSrc src{k, v, p.unit};
+  quantize_part(src, out + (int64_t)p.unit * SUB, lds, nullptr, p.kpass, p.part);
 }
 
-__global__ void __launch_bounds__(QTHREADS) flush_kernel(const uint16_t* __restrict__ ep, const int64_t* __restrict__ eoff,
+__global__ void __launch_bounds__(QTHREADS, QWPS) flush_kernel(const uint16_t* __restrict__ ep, const int64_t* __restrict__ eoff,
                                                          int64_t es, int64_t ebs, int64_t e_hs, int64_t e_ts, int64_t e_v,
                                                          uint8_t* __restrict__ qpool, const int64_t* __restrict__ qbt,
                                                          int64_t qs, int64_t bsq, int64_t qs0,
                                                          const int32_t* __restrict__ nq_prev,
                                                          const int32_t* __restrict__ nq_new, int64_t R, int max_new) {
-  __shared__ __align__(16) char lds[QLDS_BYTES];
+  __shared__ __align__(16) char lds[sizeof(QuantLds)];
   __shared__ int64_t rowtab[BLK];
-  const int64_t units = R * max_new, i = blockIdx.x;
-  const bool kpass = i < 4 * units;
-  const int64_t unit = kpass ? i / 4 : (i - 4 * units) / VSPLIT;
-  const int64_t r = unit / max_new;
-  const int j = nq_prev[r] + (int)(unit % max_new);
+  const Part p = part_of((int)R * max_new, VSPLIT);
+  const int r = p.unit / max_new;
+  const int j = nq_prev[r] + p.unit % max_new;
   if (j >= nq_new[r]) return;   // uniform over the workgroup
   const int64_t tok0 = (int64_t)j * BLK;
-  uint8_t* dst = qpool + qbt[r * qs + tok0 / bsq] * qs0 + ((tok0 % bsq) / BLK) * SUB;
-  PagedSrc src{ep, eoff + r * es, ebs, e_hs, e_ts, e_v, tok0};
-  src.prepare(rowtab);
-  quantize_part(src, dst, lds, kpass, kpass ? (int)(i % 4) : (int)((i - 4 * units) % VSPLIT));
+  uint8_t* dst = qpool + qbt[(int64_t)r * qs + tok0 / bsq] * qs0 + ((tok0 % bsq) / BLK) * SUB;
+  PagedSrc src{ep, eoff + (int64_t)r * es, ebs, e_hs, e_ts, e_v, tok0};
+  quantize_part(src, dst, lds, rowtab, p.kpass, p.part);
 }
 
 // ---------------------------------------------------------------- latency-oriented flush (decode steps)
 // A decode step flushes one or two sub-blocks per layer, so the flush costs one sub-block's latency, not throughput.
-// Same code as the throughput flush, with finer work: one token per V wave (32 V workgroups per sub-block instead of 4
-// of 64 tokens) and the K rows read 16 at a time (4 dependent round trips instead of 8).
-constexpr int LSPLIT = BLK / QW;   // V workgroups per sub-block in the latency flush: one token per wave
+// Same code as the throughput flush, with finer work: one group of four tokens per V wave (8 V workgroups per sub-block
+// instead of 4 of 64 tokens).
+constexpr int LSPLIT = BLK / (4 * QW);   // V workgroups per sub-block in the latency flush
 
 __global__ void __launch_bounds__(QTHREADS) flush_lat_kernel(const uint16_t* __restrict__ ep,
                                                              const int64_t* __restrict__ eoff, int64_t es, int64_t ebs,
@@ -484,20 +699,19 @@ __global__ void __launch_bounds__(QTHREADS) flush_lat_kernel(const uint16_t* __r
                                                              int64_t qs, int64_t bsq, int64_t qs0,
                                                              const int32_t* __restrict__ nq_prev,
                                                              const int32_t* __restrict__ nq_new, int64_t R, int max_new) {
-  __shared__ __align__(16) char lds[QLDS_BYTES];
+  __shared__ __align__(16) char lds[sizeof(QuantLds)];
   __shared__ int64_t rowtab[BLK];
-  const int64_t units = R * max_new, i = blockIdx.x;
-  const bool kpass = i < units;
-  const int64_t unit = kpass ? i : (i - units) / LSPLIT;
-  const int64_t r = unit / max_new;
-  const int j = nq_prev[r] + (int)(unit % max_new);
+  const Part p = part_of((int)R * max_new, LSPLIT);
+  const int r = p.unit / max_new;
+  const int j = nq_prev[r] + p.unit % max_new;
   if (j >= nq_new[r]) return;   // uniform over the workgroup
   const int64_t tok0 = (int64_t)j * BLK;
-  uint8_t* dst = qpool + qbt[r * qs + tok0 / bsq] * qs0 + ((tok0 % bsq) / BLK) * SUB;
-  PagedSrc src{ep, eoff + r * es, ebs, e_hs, e_ts, e_v, tok0};
-  src.prepare(rowtab);
-  if (kpass) quantize_k<PagedSrc, 16>(src, dst, lds);
-  else quantize_v<1>(src, dst, (int)((i - units) % LSPLIT) * QW, lds);
+  uint8_t* dst = qpool + qbt[(int64_t)r * qs + tok0 / bsq] * qs0 + ((tok0 % bsq) / BLK) * SUB;
+  PagedSrc src{ep, eoff + (int64_t)r * es, ebs, e_hs, e_ts, e_v, tok0};
+  if (p.kpass) {
+    src.prepare(rowtab);
+    quantize_k(src, dst, lds, p.part);
+  } else quantize_v<1>(src, dst, p.part * 4 * QW);
 }
 
 // ---------------------------------------------------------------- dequantize (kv800.py:79-92)
@@ -826,8 +1040,8 @@ int kv800_hip_flush_latency(const uint16_t* epool, const int64_t* eoff, int64_t 
   KV800_REQUIRE(ebs > 0 && bsq > 0 && bsq % BLK == 0, "flush_latency: ebs must be > 0 and bsq a positive multiple of 256");
   KV800_REQUIRE(e_hs % 8 == 0 && e_ts % 8 == 0 && e_v % 8 == 0 && ((uintptr_t)epool % 16) == 0,
                 "flush_latency: exact-pool strides must be multiples of 8 elements and the pool 16-byte aligned");
-  KV800_REQUIRE(R * max_new * (1 + LSPLIT) <= 0x7FFFFFFF, "flush_latency: grid too large");
-  hipLaunchKernelGGL(flush_lat_kernel, dim3((unsigned)(R * max_new * (1 + LSPLIT))), dim3(QTHREADS), 0,
+  KV800_REQUIRE(R * max_new * (4 + LSPLIT) <= 0x7FFFFFFF, "flush_latency: grid too large");
+  hipLaunchKernelGGL(flush_lat_kernel, dim3((unsigned)(R * max_new * (4 + LSPLIT))), dim3(QTHREADS), 0,
                      (hipStream_t)stream, epool, eoff, eoff_stride, ebs, e_hs, e_ts, e_v, qpool, qbt, qbt_stride, bsq,
                      qs0, nq_prev, nq_new, R, (int)max_new);
   return check_launch("flush_latency");

@@ -1,0 +1,87 @@
+"""The quantizer's branches on an MI355X, byte for byte against the oracle: K codes by per-channel thresholds (rounding
+near zero, constant channels, NaN channels by the arithmetic per element), V by the bounded bf16 products and by the
+exact chain (lattice values put outputs on the bit thresholds, wide ranges and infinities leave no bound to settle by),
+dense and paged, in the throughput and the latency flush."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def dev(bits):
+    return torch.from_numpy(np.ascontiguousarray(bits).view(np.int16)).view(torch.bfloat16).to(DEV)
+
+
+def draw(kind, rng, shape):
+    x = rng.standard_normal(shape)   # scales stay below fp8's largest value, 448
+    if kind == "wide":
+        x = x * np.exp2(rng.integers(-40, 4, shape))
+    elif kind == "channels":
+        x = x * np.exp2(rng.integers(-20, 5, (shape[0], 1, *shape[2:])))
+    elif kind == "lattice":
+        x = rng.integers(-6, 7, shape) * 0.25
+    elif kind == "constant":
+        x = np.broadcast_to(x[:, :1], shape) * 1.0
+    elif kind == "positive":
+        x = np.abs(x) + 0.25
+    elif kind == "cancel":
+        x[..., 64:] = -x[..., :64] * (1 + 2.0 ** -7)
+    elif kind == "near_zero":
+        x = np.where(rng.random(shape) < 0.5, x, x * np.exp(-40 * rng.random(shape)))
+    elif kind == "tiny":
+        x = x * 1e-39
+    return x.astype(np.float32)
+
+
+@pytest.mark.parametrize("kind", ["normal", "wide", "channels", "lattice", "constant", "positive", "cancel", "near_zero",
+                                  "tiny"])
+def test_quantize_kinds(hip, oracle, kind):
+    rng = np.random.default_rng(len(kind))
+    kb, vb = (oracle.f32_to_bf16(draw(kind, rng, (5, 256, 4, 128))) for _ in range(2))
+    print("quantize", kind, flush=True)
+    got = hip.quantize_blocks(dev(kb), dev(vb)).cpu().numpy()
+    assert np.array_equal(got, oracle.quantize_blocks(kb, vb))
+
+
+def test_quantize_nan_keys(hip, oracle):
+    """A NaN key is no minimum or maximum and has code 0: the bytes of the same data with the channel's minimum there."""
+    rng = np.random.default_rng(3)
+    k = draw("normal", rng, (4, 256, 4, 128))
+    holes = rng.random(k.shape) < 0.01
+    holes[0] = False                                  # a sub-block without any
+    kb, vb = oracle.f32_to_bf16(np.where(holes, np.inf, k)), oracle.f32_to_bf16(draw("normal", rng, k.shape))
+    fill = oracle.f32_to_bf16(np.where(holes, np.inf, k).min(1, keepdims=True) + np.zeros_like(k))
+    want = oracle.quantize_blocks(np.where(holes, fill, kb), vb)
+    print("quantize NaN keys", flush=True)
+    got = hip.quantize_blocks(dev(np.where(holes, np.uint16(0x7FC1), kb)), dev(vb)).cpu().numpy()
+    assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("latency", [False, True])
+@pytest.mark.parametrize("ebs", [64, 96, 640])
+def test_flush_kinds(hip, oracle, ebs, latency):
+    """Paged rows of every kind, one sub-block each, through both flushes."""
+    kinds = ["normal", "lattice", "wide", "near_zero", "constant"]
+    rng = np.random.default_rng(ebs)
+    R, pages = len(kinds), -(-640 // ebs)
+    kb, vb = (np.stack([oracle.f32_to_bf16(draw(k, rng, (1, 640, 4, 128)))[0] for k in kinds]) for _ in range(2))
+    perm = rng.permutation(R * pages).reshape(R, pages)
+    ev = np.zeros((R * pages, 4, ebs, 256), np.uint16)
+    for r in range(R):
+        for p in range(640):
+            ev[perm[r, p // ebs], :, p % ebs, :128] = kb[r, p]
+            ev[perm[r, p // ebs], :, p % ebs, 128:] = vb[r, p]
+    e = dev(ev)
+    eoff = torch.from_numpy(perm.astype(np.int64)).to(DEV) * e.stride(0)
+    qbt = torch.arange(R, device=DEV).view(R, 1)
+    j = torch.tensor([0, 1, 1, 0, 1], dtype=torch.int32, device=DEV)
+    qv = torch.zeros(R, 262144, dtype=torch.uint8, device=DEV)
+    print("flush", ebs, latency, flush=True)
+    hip.flush(e, eoff, ebs, e.stride(1), e.stride(2), 128, qv, qbt, 1280, 262144, j, j + 1, 1, latency=latency)
+    got, j = qv.cpu().numpy(), j.tolist()
+    for r in range(R):
+        s = slice(256 * j[r], 256 * j[r] + 256)
+        want = oracle.quantize_blocks(kb[r, s][None], vb[r, s][None])[0]
+        assert np.array_equal(got[r, j[r] * 51200:(j[r] + 1) * 51200], want), kinds[r]
