@@ -26,12 +26,11 @@ __device__ __forceinline__ uint32_t f2bf(float f) {
 }
 __device__ __forceinline__ float bfround(float f) { return __uint_as_float(f2bf(f) << 16); }
 
-// fp8 e4m3fn byte -> float, exact; no NaN handling (the scales the quantizer writes are finite for finite input)
+// fp8 e4m3fn byte -> float, exact; no NaN handling (the scales the quantizer writes are finite for finite input): the
+// hardware conversion, with the two NaN bytes read as the +-480 that their bits spell
 __device__ __forceinline__ float f8d(uint32_t b) {
-  const uint32_t e = (b >> 3) & 15u, m = b & 7u;
-  const uint32_t nrm = ((e + 120u) << 23) | (m << 20);
-  const uint32_t sub = __float_as_uint((float)m * 0.001953125f);
-  return __uint_as_float((e ? nrm : sub) | ((b & 0x80u) << 24));   // selects, no control flow
+  const float r = __builtin_amdgcn_cvt_f32_fp8((int)b, 0);
+  return r == r ? r : __uint_as_float(0x43F00000u | ((b & 0x80u) << 24));
 }
 
 // float -> fp8 e4m3fn byte with torch's .to(float8_e4m3fn) semantics (round to nearest even on the e4m3 grid,

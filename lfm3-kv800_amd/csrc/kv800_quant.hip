@@ -277,57 +277,9 @@ __device__ void quantize_k(const Src& src, uint8_t* __restrict__ out, char* lds,
 }
 
 // ---------------------------------------------------------------- V path
-// One lane owns 8 dims of one head row: lane = 16 hh + jj computes head hh's dims jj + 16 i (i = 0..7), which are
-// exactly the 8 bits of the row's code byte jj. For k = 16 m + kl (m, i < 8, kl < 16),
-// H[k][jj + 16 i] = H[kl][jj] (-1)^popcount(m & i), so the lane keeps the 16 values H[kl][jj] and every other sign is
-// a compile-time negation.
-__device__ __forceinline__ void hadamard_low(float (&hl)[16], int jj) {
-  const float c = __uint_as_float(0x3DB504F3u);   // fp32(1 / sqrt(128))
-#pragma unroll
-  for (int kl = 0; kl < 16; ++kl) hl[kl] = (__builtin_popcount(kl & jj) & 1) ? -c : c;
-}
-
+// For k = 16 m + kl (m, i < 8, kl < 16), H[k][j + 16 i] = H[kl][j] (-1)^popcount(m & i): a column j keeps the 16 values
+// H[kl][j] and every other sign is a compile-time negation; dims j + 16 i (i = 0..7) are the 8 bits of code byte j.
 __device__ __forceinline__ constexpr bool hneg(int m, int i) { return __builtin_popcount(m & i) & 1; }
-
-// y[i] = sum_k x[k] H[k][jj + 16 i], each output by torch-CPU's sequential fma chain over k = 0..127. Outputs whose
-// signs agree on a prefix of k share its partial sums: one chain for k < 16, two for k < 32 (by i & 1), four for
-// k < 64 (by i & 3), eight after (688 fmas for the 8 outputs instead of 1024). x (the lane's staged row) is read one
-// float4 at a time, two reads ahead of their use.
-__device__ __forceinline__ void hadamard_row8(const float* x, const float (&hl)[16], float (&y)[8]) {
-  float4 buf[3];
-  buf[0] = *reinterpret_cast<const float4*>(x);
-  buf[1] = *reinterpret_cast<const float4*>(x + 4);
-  float ch[8];
-  ch[0] = 0.f;
-#pragma unroll
-  for (int g = 0; g < 32; ++g) {   // k = 4 g .. 4 g + 3
-    if (g + 2 < 32) buf[(g + 2) % 3] = *reinterpret_cast<const float4*>(x + 4 * (g + 2));
-    const float4 v = buf[g % 3];
-    const float xv[4] = {v.x, v.y, v.z, v.w};
-    const int m = g >> 2;   // k >> 4
-    if (g == 4) ch[1] = ch[0];
-    if (g == 8) { ch[2] = ch[0]; ch[3] = ch[1]; }
-    if (g == 16) { ch[4] = ch[0]; ch[5] = ch[1]; ch[6] = ch[2]; ch[7] = ch[3]; }
-    const int nch = m == 0 ? 1 : m == 1 ? 2 : m < 4 ? 4 : 8;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const float h = hl[(4 * g + e) & 15];
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-        if (i < nch) ch[i] = __builtin_fmaf(xv[e], hneg(m, i) ? -h : h, ch[i]);
-    }
-    // the group's fmas stay before this point and the next group's reads after it: two reads ahead, no further (the
-    // live chains only; the last group's results stay plain fma results)
-    if (nch == 1) asm volatile("" : "+v"(ch[0])::"memory");
-    else if (nch == 2) asm volatile("" : "+v"(ch[0]), "+v"(ch[1])::"memory");
-    else if (nch == 4) asm volatile("" : "+v"(ch[0]), "+v"(ch[1]), "+v"(ch[2]), "+v"(ch[3])::"memory");
-    else if (g < 31)
-      asm volatile("" : "+v"(ch[0]), "+v"(ch[1]), "+v"(ch[2]), "+v"(ch[3]), "+v"(ch[4]), "+v"(ch[5]), "+v"(ch[6]),
-                   "+v"(ch[7])::"memory");
-  }
-#pragma unroll
-  for (int i = 0; i < 8; ++i) y[i] = ch[i];
-}
 
 // min(x, x of a DPP partner lane); s_nop 1 gives the two wait states a DPP read of a just-written VGPR needs
 #define KV800_MIN_DPP(x, ctrl)                                                                                \
@@ -346,40 +298,13 @@ __device__ __forceinline__ float row_min16(float x) {
   return x;
 }
 
-// Scales of one token's V rows from the 8 chain outputs y each lane holds (lane 16 hh + jj: row hh): per 2-head group g
-// (lanes 32 g .. 32 g + 31, 256 outputs) the min and max through a 16-row swap -- afterwards rows 0 / 1 hold group
-// 0's min / -max partials (lanes l, l + 16 combined), rows 2 / 3 group 1's -- and DPP row reductions; lanes q = 0..3
-// then encode lo (q even) or max(hi - lo, 1e-8) (q odd) of group q >> 1 in one pass. b8 is that byte (lanes 0..3);
-// lof, scf are the lane's group's decoded lo and scale, den = max(scf, 1e-8) the quantizer's divisor.
-struct VScales { uint32_t b8; float lof, scf, den; };
-__device__ __forceinline__ VScales v_scales(const float (&y)[8], int lane) {
-  const int q = lane & 3, g = lane >> 5;
-  const float mn = fminf(fminf(fminf(y[0], y[1]), fminf(y[2], y[3])), fminf(fminf(y[4], y[5]), fminf(y[6], y[7])));
-  const float mx = fmaxf(fmaxf(fmaxf(y[0], y[1]), fmaxf(y[2], y[3])), fmaxf(fmaxf(y[4], y[5]), fmaxf(y[6], y[7])));
-  const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(mn), __float_as_uint(-mx), false, false);
-  const float red = row_min16(vmin(__uint_as_float(sw[0]), __uint_as_float(sw[1])));
-  const float lo0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(red), 0));
-  const float hi0 = -__int_as_float(__builtin_amdgcn_readlane(__float_as_int(red), 16));
-  const float lo1 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(red), 32));
-  const float hi1 = -__int_as_float(__builtin_amdgcn_readlane(__float_as_int(red), 48));
-  const float glo = (q & 2) ? lo1 : lo0, ghi = (q & 2) ? hi1 : hi0;
-  const uint32_t b8 = f8e((q & 1) ? clamp_min_1e8(__fsub_rn(ghi, glo)) : glo);
-  const float dec = f8d(b8);
-  const float lof0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(dec), 0));
-  const float scf0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(dec), 1));
-  const float lof1 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(dec), 2));
-  const float scf1 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(dec), 3));
-  const float scf = g ? scf1 : scf0;
-  return VScales{b8, g ? lof1 : lof0, scf, clamp_min_1e8(scf)};
-}
-
 // ---------------------------------------------------------------- V path on the fp32 matrix cores
 // y = x H for 16 head rows at once (4 tokens x 4 heads; row m = 4 token + head), every output still the sequential fma
 // chain over k = 0..127: v_mfma_f32_16x16x4_f32 adds its four products to the accumulator one after another, k
 // ascending, each as one IEEE fma (denormals, infinities and NaN included; measured against the scalar chain bit for
-// bit), so 32 steps of four k make the chain. Prefixes are shared as in hadamard_row8: tile i holds dims j + 16 i
-// (column j), one tile for k < 16, two for k < 32, four for k < 64, eight after: 172 MFMA for 16 rows' 2,048 outputs.
-// Why: the part issues 75 T fp32 fma/s through MFMA and sustained 35 T through these vector chains.
+// bit), so 32 steps of four k make the chain. Outputs whose signs agree on a prefix of k share its partial sums: tile i
+// holds dims j + 16 i (column j), one tile for k < 16, two for k < 32, four for k < 64, eight after: 172 MFMA for 16
+// rows' 2,048 outputs. Why: the part issues 75 T fp32 fma/s through MFMA and sustained 35 T in vector chains.
 //   A operand: lane (g, m) = (lane / 16, lane % 16) holds x[m][4 s + g] in x[s];
 //   B operand: H[4 s + g][j] for s < 4 (the other k differ by hneg's sign), and its negation;
 //   result:    lane (g, j), y[i][r] = output j + 16 i of row 4 g + r: the lane's eight tiles at one r are the eight
@@ -392,27 +317,40 @@ __device__ __forceinline__ HadB had_operand(int lane) {
   const f4 p = {h(0), h(1), h(2), h(3)};
   return HadB{p, -p};
 }
-// conv(in[q], x) delivers x[m][4 s + g], s = 8 q .. 8 q + 7, as the chain reaches them
-template <typename T, typename Conv>
-__device__ __forceinline__ void hadamard_rows16(const T (&in)[4], Conv conv, const HadB& b, f4 (&y)[8]) {
-  y[0] = f4{0.f, 0.f, 0.f, 0.f};
+// Step S of the chain: every tile that exists for its k (templates, so that no tile is indexed at run time)
+template <int S>
+__device__ __forceinline__ void had_step(float x, const HadB& b, f4 (&y)[8]) {
+  constexpr int m = S >> 2, nch = m == 0 ? 1 : m == 1 ? 2 : m < 4 ? 4 : 8;
+  if constexpr (S == 4 || S == 8 || S == 16) {
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    float x[8];
-    conv(in[q], x);
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int s = 8 * q + u, m = s >> 2, nch = m == 0 ? 1 : m == 1 ? 2 : m < 4 ? 4 : 8;
-      if (s == 4 || s == 8 || s == 16) {
-#pragma unroll
-        for (int i = 0; i < nch / 2; ++i) y[nch / 2 + i] = y[i];
-      }
-#pragma unroll
-      for (int i = 0; i < nch; ++i)
-        y[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[u], hneg(m, i) ? b.n[s & 3] : b.p[s & 3], y[i], 0, 0, 0);
-    }
-    __builtin_amdgcn_sched_barrier(0);   // one piece's x at a time
+    for (int i = 0; i < nch / 2; ++i) y[nch / 2 + i] = y[i];
   }
+#pragma unroll
+  for (int i = 0; i < nch; ++i)
+    y[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, hneg(m, i) ? b.n[S & 3] : b.p[S & 3], y[i], 0, 0, 0);
+}
+template <int Q, typename Get>
+__device__ __forceinline__ void had_piece(const Get& get, const HadB& b, f4 (&y)[8]) {
+  float x[8];
+  get(Q, x);
+  had_step<8 * Q>(x[0], b, y);
+  had_step<8 * Q + 1>(x[1], b, y);
+  had_step<8 * Q + 2>(x[2], b, y);
+  had_step<8 * Q + 3>(x[3], b, y);
+  had_step<8 * Q + 4>(x[4], b, y);
+  had_step<8 * Q + 5>(x[5], b, y);
+  had_step<8 * Q + 6>(x[6], b, y);
+  had_step<8 * Q + 7>(x[7], b, y);
+  __builtin_amdgcn_sched_barrier(0);   // one piece's x at a time
+}
+// get(q, x) delivers x[m][4 s + g], s = 8 q .. 8 q + 7, as the chain reaches them
+template <typename Get>
+__device__ __forceinline__ void hadamard_rows16(const Get& get, const HadB& b, f4 (&y)[8]) {
+  y[0] = f4{0.f, 0.f, 0.f, 0.f};
+  had_piece<0>(get, b, y);
+  had_piece<1>(get, b, y);
+  had_piece<2>(get, b, y);
+  had_piece<3>(get, b, y);
 }
 
 // 4 x 4 transpose between four registers and the lanes l, l ^ 16, l ^ 32, l ^ 48: lane group g's register e becomes
@@ -591,7 +529,6 @@ __device__ __forceinline__ bool quick_v4(const uint4 (&in)[4], const SignB& sb, 
 // they are; for the exact chain the pieces' elements change places with the other lane groups' so
 // that the lane holds x[m][4 s + g].
 constexpr int VSPLIT = 4, VTOK = BLK / VSPLIT, VTPW = VTOK / QW;
-constexpr int VROW = 132;   // floats per staged row: the 4 rows of a token start on different LDS banks
 
 // Elements 4 u + e (u < 2, e < 4) of the 16-byte bf16 pieces 8 g' + 32 q in the lane groups g' -> lane group g's
 // x[2 g' + u] = element 4 u + g of group g', i.e. k = 4 (8 q + 2 g' + u) + g
@@ -622,7 +559,7 @@ __device__ void quantize_v(const Src& src, uint8_t* __restrict__ out, int t0) {
     uint32_t b8, w;
     if (!quick_v4(in, sb, lane, b8, w)) {   // uniform over the wave
       f4 y[8];
-      hadamard_rows16(in, unpack_piece, had_operand(lane), y);
+      hadamard_rows16([&](int q, float (&x)[8]) { unpack_piece(in[q], x); }, had_operand(lane), y);
       const VScales4 sc = v_scales4(y, lane);
       b8 = sc.b8;
       w = v_bits4(y, sc);
@@ -635,9 +572,10 @@ __device__ void quantize_v(const Src& src, uint8_t* __restrict__ out, int t0) {
 
 // A quantize grid holds, per sub-block, VSPLIT V workgroups (V is independent per token) and 4 K workgroups (one per
 // head: all 256 tokens per channel, each row read once). All V workgroups come first: they are the long ones, and the K
-// workgroups fill in behind them (448 sub-blocks: 91 us, 98-118 us interleaved, 100 us with K first). V alone takes
-// 65 us, K alone 40 us, both mostly the latency of one-shot workgroups at two per CU; 448 sub-blocks of paged rows took
-// 147 us with a scalar fma chain per V lane and the code arithmetic per K element, and take 90 us now (2.9 TB/s).
+// workgroups fill in behind them (448 sub-blocks: 90 us, 98-118 us interleaved, 100 us with K first, before the chain's tiles were
+// indexed at compile time). V alone takes about 60 us, K alone 40 us, both mostly the latency of one-shot workgroups at
+// two per CU; 448 sub-blocks of paged rows took 147 us with a scalar fma chain per V lane and the code arithmetic per K
+// element, and take 84 us now (3.1 TB/s).
 // 32-bit throughout (the host bounds the grid): scalar compares and selects.
 struct Part { int unit; bool kpass; int part; };
 __device__ __forceinline__ Part part_of(int units, int vsplit) {
@@ -715,58 +653,104 @@ __global__ void __launch_bounds__(QTHREADS) flush_lat_kernel(const uint16_t* __r
 }
 
 // ---------------------------------------------------------------- dequantize (kv800.py:79-92)
-__global__ void __launch_bounds__(256) dequant_kernel(const uint8_t* __restrict__ sb, uint16_t* __restrict__ kout,
-                                                      float* __restrict__ vout) {
-  __shared__ __align__(16) float xbuf[4][4 * VROW];   // per wave: one token's 4 V rows
-  const int64_t m = blockIdx.x;
-  const uint8_t* s = sb + m * SUB;
-  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-  // K: bf16(code * ksc + klo) (product and sum rounded separately, as the reference's torch ops)
-  for (int i = tid; i < BLK * 512 / 8; i += 256) {
-    const int t = i / 64, hc0 = (i % 64) * 8, hh = hc0 >> 7, d0 = hc0 & 127;
-    uint32_t o[4];
-#pragma unroll
-    for (int e = 0; e < 8; e += 2) {
-      uint32_t pr = 0;
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const int d = d0 + e + u;
-        const uint32_t code = (s[KC_O + (t * 4 + hh) * 32 + (d & 31)] >> (2 * (d >> 5))) & 3u;
-        const float kv = __fadd_rn(__fmul_rn((float)code, f8d(s[KSC_O + hh * 128 + d])), f8d(s[KLO_O + hh * 128 + d]));
-        pr |= f2bf(kv) << (16 * u);
-      }
-      o[e >> 1] = pr;
-    }
-    *reinterpret_cast<uint4*>(kout + (m * BLK + t) * 512 + hc0) = make_uint4(o[0], o[1], o[2], o[3]);
-  }
-  // V: (bit * vsc + vlo) @ H, wave w = tokens 64w .. 64w + 63, per token its 4 head rows staged in the wave's LDS
-  // rows; lane 16 hh + jj builds dims 8 jj .. 8 jj + 7 of row hh and gets dims jj + 16 i back from the chain
-  float hl[16];
-  const int hh = lane >> 4, jj = lane & 15;
-  hadamard_low(hl, jj);
-  float* xrow = &xbuf[w][hh * VROW];
-  for (int tt = 0; tt < 64; ++tt) {
-    const int t = 64 * w + tt;
-    {
-      const float vsc = f8d(s[VSC_O + t * 2 + (hh >> 1)]), vlo = f8d(s[VLO_O + t * 2 + (hh >> 1)]);
-      const uint8_t* vb = s + VB_O + (t * 4 + hh) * 16;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int d = 8 * jj + e;
-        const float bit = (float)((vb[d & 15] >> (d >> 4)) & 1u);
-        xrow[d] = __fadd_rn(__fmul_rn(bit, vsc), vlo);
-      }
-    }
-    __builtin_amdgcn_wave_barrier();   // a wave's LDS instructions run in order: this token's rows, then its reads
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    float y[8];
-    hadamard_row8(xrow, hl, y);
-    float* vo = vout + ((m * BLK + t) * 4 + hh) * 128 + jj;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) vo[16 * i] = y[i];
-  }
+// Loads of sub-block bytes wherever the caller's sub-blocks start (the hardware takes any alignment)
+struct __attribute__((packed, aligned(1))) Bytes16 { uint32_t x, y, z, w; };
+struct __attribute__((packed, aligned(1))) Bytes8 { uint32_t x, y; };
+__device__ __forceinline__ uint4 load16(const uint8_t* p) {
+  const Bytes16 b = *reinterpret_cast<const Bytes16*>(p);
+  return make_uint4(b.x, b.y, b.z, b.w);
+}
+__device__ __forceinline__ uint2 load8(const uint8_t* p) {
+  const Bytes8 b = *reinterpret_cast<const Bytes8*>(p);
+  return make_uint2(b.x, b.y);
 }
 
+// V rows back from their bits: y = (bit vsc + vlo) H for four tokens x 4 heads by the exact chain. Lane (g, m) holds row
+// m's 16 code bytes and its two values; step s = 4 i + a takes bit i of byte 4 a + g.
+__device__ __forceinline__ void dequant_rows16(const uint4& vb, float vsc, float vlo, const HadB& hb, int g, f4 (&y)[8]) {
+  const uint32_t lo = __float_as_uint(__fadd_rn(__fmul_rn(0.f, vsc), vlo)), hi = __float_as_uint(__fadd_rn(vsc, vlo));
+  const uint32_t b0 = (vb.x >> (8 * g)) & 0xFFu, b1 = (vb.y >> (8 * g)) & 0xFFu;
+  const uint32_t b2 = (vb.z >> (8 * g)) & 0xFFu, b3 = (vb.w >> (8 * g)) & 0xFFu;
+  auto pick = [&](uint32_t b, int i) {
+    const uint32_t mask = (uint32_t)((int32_t)(b << (31 - i)) >> 31);
+    return __uint_as_float((mask & hi) | (~mask & lo));
+  };
+  hadamard_rows16(
+      [&](int q, float (&x)[8]) {
+#pragma unroll
+        for (int ii = 0; ii < 2; ++ii) {
+          x[4 * ii] = pick(b0, 2 * q + ii);
+          x[4 * ii + 1] = pick(b1, 2 * q + ii);
+          x[4 * ii + 2] = pick(b2, 2 * q + ii);
+          x[4 * ii + 3] = pick(b3, 2 * q + ii);
+        }
+      },
+      hb, y);
+}
+
+// Two rounded dequantized keys, packed: bf16(code sc + lo) of byte E of the codes c (the product is exact in fp32, so
+// the fused multiply-add rounds where torch's add does); v_cvt_pk_bf16_f32 rounds as f2bf for finite values.
+typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t bfpk(float a, float b) {
+  const bf2 v = {(__bf16)a, (__bf16)b};
+  return __builtin_bit_cast(uint32_t, v);
+}
+__device__ __forceinline__ float ubyte(uint32_t c, int e) { return (float)((c >> (8 * e)) & 0xFFu); }   // one conversion
+
+// One workgroup per quarter of a sub-block and side (its K, its V), so that 448 sub-blocks fill the part and the V
+// chains' workgroups run beside the K workgroups' stores. K: a lane keeps its 8 channels' scales in registers and a
+// wave writes whole 1 KB token rows. 448 sub-blocks: 205 us as one workgroup per sub-block with per-element scale
+// reads and vector chains, 122 us now (3.1 TB/s).
+constexpr int DPARTS = 4, DTOK = BLK / DPARTS;
+__global__ void __launch_bounds__(256) dequant_kernel(const uint8_t* __restrict__ sb, int M, uint16_t* __restrict__ kout,
+                                                      float* __restrict__ vout) {
+  const int i = (int)blockIdx.x, nv = DPARTS * M;
+  const bool kside = i >= nv;                       // V workgroups, the longer ones, first
+  const int o = kside ? i - nv : i;
+  const int64_t mb = o / DPARTS;
+  const uint8_t* s = sb + mb * SUB;
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, t0 = (o % DPARTS) * DTOK;
+  if (kside) {
+    const int h = lane >> 4, p = (lane >> 2) & 3, q = lane & 3, hc0 = 8 * lane;   // dims 32 p + 8 q .. + 7 of head h
+    float sc[8], lo[8];
+    {
+      const uint2 a = load8(s + KSC_O + hc0), b = load8(s + KLO_O + hc0);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        sc[e] = f8d(((e < 4 ? a.x : a.y) >> (8 * (e & 3))) & 0xFFu);
+        lo[e] = f8d(((e < 4 ? b.x : b.y) >> (8 * (e & 3))) & 0xFFu);
+      }
+    }
+    const uint8_t* kc = s + KC_O + ((t0 + w) * 4 + h) * 32 + 8 * q;
+    uint16_t* ko = kout + (mb * BLK + t0 + w) * 512 + hc0;
+#pragma unroll 4
+    for (int t = 0; t < DTOK; t += 4) {
+      const uint2 by = load8(kc + t * 128);
+      const uint32_t c0 = (by.x >> (2 * p)) & 0x03030303u, c1 = (by.y >> (2 * p)) & 0x03030303u;
+      uint4 r;
+      r.x = bfpk(__builtin_fmaf(ubyte(c0, 0), sc[0], lo[0]), __builtin_fmaf(ubyte(c0, 1), sc[1], lo[1]));
+      r.y = bfpk(__builtin_fmaf(ubyte(c0, 2), sc[2], lo[2]), __builtin_fmaf(ubyte(c0, 3), sc[3], lo[3]));
+      r.z = bfpk(__builtin_fmaf(ubyte(c1, 0), sc[4], lo[4]), __builtin_fmaf(ubyte(c1, 1), sc[5], lo[5]));
+      r.w = bfpk(__builtin_fmaf(ubyte(c1, 2), sc[6], lo[6]), __builtin_fmaf(ubyte(c1, 3), sc[7], lo[7]));
+      *reinterpret_cast<uint4*>(ko + (int64_t)t * 512) = r;
+    }
+    return;
+  }
+  const int g = lane >> 4, m = lane & 15;
+  const HadB hb = had_operand(lane);
+#pragma unroll 1
+  for (int t = t0 + 4 * w; t < t0 + DTOK; t += 16) {
+    const int tm = t + (m >> 2);
+    const uint4 vb = load16(s + VB_O + tm * 64 + (m & 3) * 16);
+    f4 y[8];
+    dequant_rows16(vb, f8d(s[VSC_O + tm * 2 + ((m >> 1) & 1)]), f8d(s[VLO_O + tm * 2 + ((m >> 1) & 1)]), hb, g, y);
+    float* vo = vout + (mb * BLK + t + g) * 512 + m;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int i8 = 0; i8 < 8; ++i8) vo[r * 128 + 16 * i8] = y[i8][r];
+  }
+}
 
 // ---------------------------------------------------------------- training fake quantization (train.py:82-100)
 // fake_quant_k: x (G, 256, C) fp32 -> c * sc8 + lo8 per (group, channel), the K path of the quantizer on fp32 input
@@ -798,45 +782,54 @@ __global__ void __launch_bounds__(256) fake_quant_k_kernel(const float* __restri
 
 // fake_quant_v: v (N, 4, 128) fp32 -> per token y = v H (the quantizer's sequential fma chain), one bit per dim with
 // fp8 lo / scale per pair of heads, then (bit * sc8 + lo8) H with the dequantizer's chain: the V value of a
-// quantize -> dequantize round trip. One wave per token at a time, the token's rows staged in LDS; lane 16 hh + jj
-// holds dims jj + 16 i of row hh in both chains (the quantizer's scales and bit test as in quantize_v).
-constexpr int FQV_TPW = 8;   // tokens per wave
+// quantize -> dequantize round trip. A wave takes four tokens at a time through both chains on fp32 MFMA; lane (g, m)
+// loads the float4s 4 (4 u + g) of row m, whose elements change places with the other lane groups'. Between the chains
+// the code bytes and the scales go from the result's lanes to the next operand's through the wave's 320 bytes of LDS.
+// 32,768 tokens: 67 us with vector chains, 59 us now; bound: 42 us of fp32 MFMA beside the scales and bits on the VALU.
+constexpr int FQV_GROUPS = 2;   // groups of four tokens per wave
+struct FqvLds { uint32_t vb[16][4]; float sc[4][4]; };   // row's code bytes; token's (lo, scale) per pair of heads
 __global__ void __launch_bounds__(256) fake_quant_v_kernel(const float* __restrict__ v, int64_t N,
                                                            float* __restrict__ out) {
-  __shared__ __align__(16) float xb[4][4 * VROW];   // per wave: the token's 4 rows (v, then the dequantized values)
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int hh = lane >> 4, jj = lane & 15;
-  float hl[16];
-  hadamard_low(hl, jj);
-  float* xrow = &xb[w][hh * VROW];
-  const int64_t t0 = ((int64_t)blockIdx.x * 4 + w) * FQV_TPW;
+  __shared__ FqvLds xb[4];
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, m = lane & 15;
+  FqvLds& L = xb[w];
+  const HadB hb = had_operand(lane);
 #pragma unroll 1
-  for (int tt = 0; tt < FQV_TPW; ++tt) {
-    const int64_t t = t0 + tt;
+  for (int gr = 0; gr < FQV_GROUPS; ++gr) {
+    const int64_t t = (((int64_t)blockIdx.x * 4 + w) * FQV_GROUPS + gr) * 4;
     if (t >= N) break;   // uniform over the wave
-    const float4* src = reinterpret_cast<const float4*>(v + (t * 4 + hh) * 128 + 8 * jj);
-    const float4 a = src[0], b = src[1];
-    *reinterpret_cast<float4*>(xrow + 8 * jj) = a;
-    *reinterpret_cast<float4*>(xrow + 8 * jj + 4) = b;
+    const int64_t tm = min(t + (m >> 2), N - 1);   // rows past the end repeat the last token's and are not stored
+    const float4* src = reinterpret_cast<const float4*>(v + (tm * 4 + (m & 3)) * 128) + g;
+    float4 in[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) in[u] = src[4 * u];
+    f4 y[8];
+    hadamard_rows16(
+        [&](int q, float (&x)[8]) {
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            float4 f = in[2 * q + u];
+            transpose_rows4(f.x, f.y, f.z, f.w);
+            x[4 * u] = f.x; x[4 * u + 1] = f.y; x[4 * u + 2] = f.z; x[4 * u + 3] = f.w;
+          }
+        },
+        hb, y);
+    const VScales4 sc = v_scales4(y, lane);
+    L.vb[4 * g + (m & 3)][m >> 2] = quad_bytes(v_bits4(y, sc), lane);
+    if (m == 0) *reinterpret_cast<float4*>(L.sc[g]) = make_float4(sc.lof[0], sc.scf[0], sc.lof[1], sc.scf[1]);
     __builtin_amdgcn_wave_barrier();   // a wave's LDS instructions run in order
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    float y[8];
-    hadamard_row8(xrow, hl, y);
-    const VScales sc = v_scales(y, lane);
-    const float half = sc.den * 0.5f;
-    float z[8];
+    const uint4 vb = *reinterpret_cast<const uint4*>(L.vb[m]);
+    const float2 ls = *reinterpret_cast<const float2*>(&L.sc[m >> 2][m & 2]);
+    __builtin_amdgcn_wave_barrier();   // and the next group's writes follow these reads
+    dequant_rows16(vb, ls.y, ls.x, hb, g, y);
+    if (t + g < N) {
+      float* vo = out + (t + g) * 512 + m;
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-      z[i] = __fadd_rn(__fmul_rn((__fsub_rn(y[i], sc.lof) > half) ? 1.f : 0.f, sc.scf), sc.lof);
-    __builtin_amdgcn_wave_barrier();   // every lane has read the v rows
+      for (int r = 0; r < 4; ++r)
 #pragma unroll
-    for (int i = 0; i < 8; ++i) xrow[jj + 16 * i] = z[i];
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    hadamard_row8(xrow, hl, y);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) out[(t * 4 + hh) * 128 + jj + 16 * i] = y[i];
-    __builtin_amdgcn_wave_barrier();   // the next token's rows overwrite the staged rows
+        for (int i = 0; i < 8; ++i) vo[r * 128 + 16 * i] = y[i][r];
+    }
   }
 }
 
@@ -847,10 +840,10 @@ __global__ void __launch_bounds__(256) fake_quant_v_kernel(const float* __restri
 // dequantizer's fp32 chain, then bf16: dequantize_blocks, kv800.py:79-92), the others from the exact pages. RoPE is the
 // reference's fp32 kf c + rotate_half(kf) s over the 128-wide tables (cos32 | 1 | cos32 | 1), (sin32 | 0 | sin32 | 0),
 // each product and the sum rounded once, then bf16. Unreadable rows (offsets outside their pool, positions past the
-// rope table) are written as zeros. One workgroup per (hpos-position tile, row): hpos = 64, a quarter of a sub-block,
-// so that the V chain (one wave per token at a time) runs at eight waves per SIMD on a long prefill, or 16 or 4 when
-// 64 gives fewer than 1,024 workgroups (a single row). hpos divides 256, so a tile never straddles a sub-block; the
-// outputs do not depend on it.
+// rope table) are written as zeros. One workgroup per (hpos-position tile, row): hpos = 32 (two MFMA groups of four
+// tokens per wave), or 16 when 32 gives fewer than 1,024 workgroups (a single row). hpos divides 256, so a tile never
+// straddles a sub-block; the outputs do not depend on it. 8 rows of 16K positions: 212 us with vector chains and
+// software rounding, 134 us now (64 or 16 positions: 137 / 144 us); one row 48 -> 24 us. Bound: 84 us of fp32 MFMA.
 __device__ __forceinline__ void rope8(float (&a)[8], float (&b)[8], const uint16_t* cs, const uint16_t* sn, bool rope) {
   // a = dims d0 .. d0 + 7, b = dims d0 + 64 .. d0 + 71; rope: d0 < 32 (cs / sn the tables' entries d0 ..), else the
   // unrotated dims, for which the table holds cos 1, sin 0
@@ -867,16 +860,13 @@ __device__ __forceinline__ uint4 pack_bf16x8(const float (&x)[8]) {
                     f2bf(x[6]) | (f2bf(x[7]) << 16));
 }
 
-// positions per history workgroup: a quarter of a sub-block, cut by 4 (down to 4 positions, one token per wave)
-// while the rows give fewer than four workgroups per CU (a single long row: the V chain then runs at four waves per
-// SIMD instead of one)
-constexpr int HPOS = 64, HPOS_MIN = 4, HPOS_MIN_GROUPS = 1024;
+// positions per history workgroup
+constexpr int HPOS = 32, HPOS_MIN = 16, HPOS_MIN_GROUPS = 1024;
 __global__ void __launch_bounds__(256) history_kernel(kv800_paged_t P, const uint16_t* __restrict__ cos_t,
                                                       const uint16_t* __restrict__ sin_t, int64_t rope_rows,
                                                       int64_t qpool_bytes, int64_t epool_elems,
                                                       const int64_t* __restrict__ out_off, uint16_t* __restrict__ kout,
                                                       uint16_t* __restrict__ vout, int hpos) {
-  __shared__ __align__(16) float xbuf[4][4 * VROW];   // per wave: one token's 4 dequantized V rows
   __shared__ float klo_s[512], ksc_s[512];
   const int r = blockIdx.y, tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
   const int n = P.N[r], p0 = blockIdx.x * hpos;
@@ -891,62 +881,93 @@ __global__ void __launch_bounds__(256) history_kernel(kv800_paged_t P, const uin
     const int64_t base = P.boff[(int64_t)r * P.boff_stride + sb];
     const bool ok = base >= 0 && base + SUB <= qpool_bytes;   // uniform
     const uint8_t* s = P.qpool + (ok ? base : 0);
+    bool neg = false;   // a negative scale (the quantizer writes none) can give a key -0
     if (ok)
-      for (int i = tid; i < 512; i += 256) { klo_s[i] = f8d(s[KLO_O + i]); ksc_s[i] = f8d(s[KSC_O + i]); }
-    __syncthreads();
-    // K: unit u = (token t, head h, d0 = 8 (u % 8)): dims d0 .. d0 + 7 and d0 + 64 .. d0 + 71
-    for (int u = tid; u < cnt * 32; u += 256) {
-      const int t = u >> 5, h = (u >> 3) & 3, d0 = 8 * (u & 7);
-      uint16_t* ko = kout + (ob + t) * 512 + h * 128 + d0;
+      for (int i = tid; i < 512; i += 256) {
+        klo_s[i] = f8d(s[KLO_O + i]);
+        ksc_s[i] = f8d(s[KSC_O + i]);
+        neg |= s[KSC_O + i] > 0x7F;
+      }
+    neg = __syncthreads_or(neg);
+    // K: unit = (token t, head h, q): the code bytes 8 q .. 8 q + 7 of (t, h) give dims 32 k + 8 q .. + 7, k = 0..3, of
+    // which k = 0 and 2 are rotated
+    for (int u = tid; u < cnt * 16; u += 256) {
+      const int t = u >> 4, h = (u >> 2) & 3, q = u & 3;
+      uint16_t* ko = kout + (ob + t) * 512 + h * 128 + 8 * q;
       const int pos = p0 + t;
       if (!ok || (rot && pos >= rope_rows)) {
-        *reinterpret_cast<uint4*>(ko) = zero4;
-        *reinterpret_cast<uint4*>(ko + 64) = zero4;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) *reinterpret_cast<uint4*>(ko + 32 * k) = zero4;
         continue;
       }
-      const uint2 by = *reinterpret_cast<const uint2*>(s + KC_O + ((to + t) * 4 + h) * 32 + (d0 & 31));
-      const uint32_t bw[2] = {by.x, by.y};
-      const int sa = 2 * (d0 >> 5), sb = sa + 4;   // code fields of dims d0 + e and d0 + 64 + e
-      float a[8], b[8];
+      const uint2 by = load8(s + KC_O + ((to + t) * 4 + h) * 32 + 8 * q);
+      uint32_t o[4][4];   // dims 32 k + 8 q .. + 7, packed pairs
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const uint32_t byte = (bw[e >> 2] >> (8 * (e & 3))) & 0xFFu;
-        const int ia = h * 128 + d0 + e, ib = ia + 64;
-        a[e] = bf2f(f2bf(__fadd_rn(__fmul_rn((float)((byte >> sa) & 3u), ksc_s[ia]), klo_s[ia])));
-        b[e] = bf2f(f2bf(__fadd_rn(__fmul_rn((float)((byte >> sb) & 3u), ksc_s[ib]), klo_s[ib])));
-      }
-      if (rot) rope8(a, b, cos_t + (int64_t)pos * 32 + d0, sin_t + (int64_t)pos * 32 + d0, d0 < 32);
-      *reinterpret_cast<uint4*>(ko) = pack_bf16x8(a);
-      *reinterpret_cast<uint4*>(ko + 64) = pack_bf16x8(b);
-    }
-    // V: wave w takes tokens w, w + 4, ...; lane 16 hh + jj builds dims 8 jj .. 8 jj + 7 of bit vsc + vlo for row hh,
-    // then gets dims jj + 16 i of that row from the chain
-    float hl[16];
-    const int hh = lane >> 4, jj = lane & 15;
-    hadamard_low(hl, jj);
-    float* xrow = &xbuf[w][hh * VROW];
-    for (int t = w; t < cnt; t += 4) {
-      uint16_t* vo = vout + (ob + t) * 512;
-      if (!ok) {
-        for (int i = lane; i < 512; i += 64) vo[i] = 0;
-        continue;
-      }
-      {
-        const float vsc = f8d(s[VSC_O + (to + t) * 2 + (hh >> 1)]), vlo = f8d(s[VLO_O + (to + t) * 2 + (hh >> 1)]);
-        const uint8_t* vb = s + VB_O + ((to + t) * 4 + hh) * 16;
+      for (int k = 0; k < 4; ++k) {
+        const float* sc = ksc_s + h * 128 + 32 * k + 8 * q;
+        const float* lo = klo_s + h * 128 + 32 * k + 8 * q;
+        const uint32_t c0 = (by.x >> (2 * k)) & 0x03030303u, c1 = (by.y >> (2 * k)) & 0x03030303u;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int d = 8 * jj + e;
-          const float bit = (float)((vb[d & 15] >> (d >> 4)) & 1u);
-          xrow[d] = __fadd_rn(__fmul_rn(bit, vsc), vlo);
+        for (int e = 0; e < 4; ++e) {
+          const uint32_t c = e < 2 ? c0 : c1;
+          const int b = 2 * (e & 1);
+          o[k][e] = bfpk(__builtin_fmaf(ubyte(c, b), sc[2 * e], lo[2 * e]),
+                         __builtin_fmaf(ubyte(c, b + 1), sc[2 * e + 1], lo[2 * e + 1]));
         }
       }
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-      float y[8];
-      hadamard_row8(xrow, hl, y);
+      if (rot) {
+        const uint4 cv = *reinterpret_cast<const uint4*>(cos_t + (int64_t)pos * 32 + 8 * q);
+        const uint4 sv = *reinterpret_cast<const uint4*>(sin_t + (int64_t)pos * 32 + 8 * q);
+        const uint32_t cw[4] = {cv.x, cv.y, cv.z, cv.w}, sw[4] = {sv.x, sv.y, sv.z, sv.w};
 #pragma unroll
-      for (int i = 0; i < 8; ++i) vo[hh * 128 + jj + 16 * i] = (uint16_t)f2bf(y[i]);
+        for (int e = 0; e < 4; ++e) {
+          const float x0 = bf2f_lo(o[0][e]), x1 = bf2f_hi(o[0][e]), y0 = bf2f_lo(o[2][e]), y1 = bf2f_hi(o[2][e]);
+          const float c0 = bf2f_lo(cw[e]), c1 = bf2f_hi(cw[e]), s0 = bf2f_lo(sw[e]), s1 = bf2f_hi(sw[e]);
+          o[0][e] = bfpk(__fadd_rn(__fmul_rn(x0, c0), __fmul_rn(-y0, s0)), __fadd_rn(__fmul_rn(x1, c1), __fmul_rn(-y1, s1)));
+          o[2][e] = bfpk(__fadd_rn(__fmul_rn(y0, c0), __fmul_rn(x0, s0)), __fadd_rn(__fmul_rn(y1, c1), __fmul_rn(x1, s1)));
+          if (neg) {   // the other dims' rotation by cos 1, sin 0 changes nothing but the sign of such a zero
+            const float a0 = bf2f_lo(o[1][e]), a1 = bf2f_hi(o[1][e]), b0 = bf2f_lo(o[3][e]), b1 = bf2f_hi(o[3][e]);
+            o[1][e] = bfpk(__fadd_rn(a0, __fmul_rn(-b0, 0.f)), __fadd_rn(a1, __fmul_rn(-b1, 0.f)));
+            o[3][e] = bfpk(__fadd_rn(b0, __fmul_rn(a0, 0.f)), __fadd_rn(b1, __fmul_rn(a1, 0.f)));
+          }
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) *reinterpret_cast<uint4*>(ko + 32 * k) = make_uint4(o[k][0], o[k][1], o[k][2], o[k][3]);
+    }
+    // V: wave w takes four tokens at a time through the dequantizer's chain; the quads' 4 x 4 exchange of packed pairs
+    // leaves each lane four consecutive dims per store
+    const int g = lane >> 4, m = lane & 15, e = m & 3;
+    const HadB hb = had_operand(lane);
+    for (int t = 4 * w; t < cnt; t += 16) {
+      const int tm = to + min(t + (m >> 2), cnt - 1);   // rows past the end repeat the last one and are not stored
+      uint4 vb = zero4;
+      float vsc = 0.f, vlo = 0.f;
+      if (ok) {
+        vb = load16(s + VB_O + tm * 64 + (m & 3) * 16);
+        vsc = f8d(s[VSC_O + tm * 2 + ((m >> 1) & 1)]);
+        vlo = f8d(s[VLO_O + tm * 2 + ((m >> 1) & 1)]);
+      }
+      f4 y[8];
+      dequant_rows16(vb, vsc, vlo, hb, g, y);   // zeros where the sub-block is not readable
+      uint16_t* vo = vout + (ob + t + g) * 512 + (m & ~3);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        uint32_t v[4];
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+          const uint32_t x = bfpk(y[2 * p][r], y[2 * p + 1][r]);
+          v[p] = __builtin_amdgcn_perm(x, quad<QUAD_X1>(x), (e & 1) ? 0x07060302u : 0x01000504u);
+        }
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {   // plane 4 p + e, dims m & ~3 .. + 3
+          const uint32_t own = (e & 2) ? v[2 * p + 1] : v[2 * p];
+          const uint32_t got = quad<QUAD_X2>((e & 2) ? v[2 * p] : v[2 * p + 1]);
+          if (t + g < cnt)
+            *reinterpret_cast<uint2*>(vo + r * 128 + 16 * (4 * p + e)) =
+                (e & 2) ? make_uint2(got, own) : make_uint2(own, got);
+        }
+      }
     }
     return;
   }
@@ -1052,9 +1073,10 @@ int kv800_hip_dequantize_blocks(const uint8_t* sb, int64_t M, uint16_t* k_out, f
   KV800_REQUIRE(M >= 0, "dequantize_blocks: M = %lld < 0", (long long)M);
   if (M == 0) return KV800_OK;
   KV800_REQUIRE(sb && k_out && v_out, "dequantize_blocks: null pointer");
-  KV800_REQUIRE(M <= 0x7FFFFFFF, "dequantize_blocks: M too large");
+  KV800_REQUIRE(M <= 0x7FFFFFFF / (2 * DPARTS), "dequantize_blocks: M too large");
   KV800_REQUIRE(((uintptr_t)k_out % 16) == 0, "dequantize_blocks: k_out must be 16-byte aligned");
-  hipLaunchKernelGGL(dequant_kernel, dim3((unsigned)M), dim3(256), 0, (hipStream_t)stream, sb, k_out, v_out);
+  hipLaunchKernelGGL(dequant_kernel, dim3((unsigned)(M * 2 * DPARTS)), dim3(256), 0, (hipStream_t)stream, sb, (int)M, k_out,
+                     v_out);
   return check_launch("dequantize_blocks");
 }
 
@@ -1075,7 +1097,7 @@ int kv800_hip_fake_quant_v(const float* v, int64_t N, float* out, void* stream) 
   if (N == 0) return KV800_OK;
   KV800_REQUIRE(v && out, "fake_quant_v: null pointer");
   KV800_REQUIRE(((uintptr_t)v % 16) == 0, "fake_quant_v: v must be 16-byte aligned");
-  const int64_t nb = (N + 4 * FQV_TPW - 1) / (4 * FQV_TPW);
+  const int64_t nb = (N + 16 * FQV_GROUPS - 1) / (16 * FQV_GROUPS);
   KV800_REQUIRE(nb <= 0x7FFFFFFF, "fake_quant_v: N too large");
   hipLaunchKernelGGL(fake_quant_v_kernel, dim3((unsigned)nb), dim3(256), 0, (hipStream_t)stream, v, N, out);
   return check_launch("fake_quant_v");
@@ -1095,7 +1117,7 @@ int kv800_hip_history(const kv800_paged_t* P, int64_t R, int64_t max_n, const ui
   KV800_REQUIRE(((uintptr_t)k_out % 16) == 0 && ((uintptr_t)v_out % 16) == 0, "history: outputs must be 16-byte aligned");
   KV800_REQUIRE(R <= 65535, "history: at most 65535 rows per call");
   int hpos = HPOS;
-  while (hpos > HPOS_MIN && (max_n + hpos - 1) / hpos * R < HPOS_MIN_GROUPS) hpos /= 4;
+  while (hpos > HPOS_MIN && (max_n + hpos - 1) / hpos * R < HPOS_MIN_GROUPS) hpos /= 2;
   const int64_t tiles = (max_n + hpos - 1) / hpos;
   KV800_REQUIRE(tiles <= 0x7FFFFFFF, "history: max_n too large");
   hipLaunchKernelGGL(history_kernel, dim3((unsigned)tiles, (unsigned)R), dim3(256), 0, (hipStream_t)stream, *P, cos_t,

@@ -85,3 +85,26 @@ def test_flush_kinds(hip, oracle, ebs, latency):
         s = slice(256 * j[r], 256 * j[r] + 256)
         want = oracle.quantize_blocks(kb[r, s][None], vb[r, s][None])[0]
         assert np.array_equal(got[r, j[r] * 51200:(j[r] + 1) * 51200], want), kinds[r]
+
+
+@pytest.mark.parametrize("blocks,shift", [(1, 0), (3, 1), (2, 12)])
+def test_dequantize_anywhere(hip, oracle, blocks, shift):
+    """Sub-blocks at any byte of their storage."""
+    rng = np.random.default_rng(shift)
+    sb = oracle.quantize_blocks(*(oracle.f32_to_bf16(draw("normal", rng, (blocks, 256, 4, 128))) for _ in range(2)))
+    raw = torch.zeros(blocks * 51200 + 16, dtype=torch.uint8, device=DEV)
+    at = raw[shift:shift + blocks * 51200].view(blocks, 51200)
+    at.copy_(torch.from_numpy(sb))
+    print("dequantize", blocks, shift, flush=True)
+    k, v = hip.dequantize_blocks(at)
+    kw, vw = oracle.dequantize_blocks(sb)
+    assert np.array_equal(k.cpu().view(torch.int16).numpy().view(np.uint16), kw)
+    assert np.array_equal(v.cpu().numpy(), vw)
+
+
+@pytest.mark.parametrize("tokens", [1, 3, 5, 33, 64])
+def test_fake_quant_v_counts(hip, oracle, tokens):
+    """Token counts around the groups of four and the waves' two groups."""
+    v = draw("normal", np.random.default_rng(tokens), (tokens, 4, 128)) * np.float32(1.7)
+    print("fake_quant_v", tokens, flush=True)
+    assert np.array_equal(hip.fake_quant_v(torch.from_numpy(v).to(DEV)).cpu().numpy(), oracle.fake_quant_v(v))
