@@ -148,6 +148,25 @@ int kv800_hip_history(const kv800_paged_t* P, int64_t R, int64_t max_n, const ui
                       int64_t rope_rows, int64_t qpool_bytes, int64_t epool_elems, const int64_t* out_off,
                       uint16_t* k_out, uint16_t* v_out, void* stream);
 
+/* All keys of a quantized layer's prefill rows in one launch: kv800_hip_history of prev[r] positions per row to output
+ * rows ksl[r] + p, followed by the chunk's new rows [qsl[r], qsl[r + 1]) of k / v ((T, 4, 128) bf16, pre-RoPE keys),
+ * rotated at positions prev[r] + i as kv800_hip_rope_rows rotates, at output rows ksl[r] + prev[r] + i (the assembly of
+ * vllm_attn.py:351-402). prev (R,), qsl and ksl (R + 1,) int64 on the device; max_prev / max_new their host bounds. */
+int kv800_hip_prefill_keys(const kv800_paged_t* P, int64_t R, int64_t max_prev, int64_t max_new, const uint16_t* cos_t,
+                           const uint16_t* sin_t, int64_t rope_rows, int64_t qpool_bytes, int64_t epool_elems,
+                           const int64_t* prev, const int64_t* qsl, const int64_t* ksl, const uint16_t* k,
+                           const uint16_t* v, uint16_t* k_out, uint16_t* v_out, void* stream);
+
+/* The same for a window layer: row r's keys are its sinks (positions < min(nsink, lo), blocks of [4, 4, 128] at
+ * P->skoff / P->svoff), its exact rows [lo, prev[r]) with lo = max(0, prev[r] - (P->win - 1)), then its new rows, at output
+ * rows ksl[r] + i, max_rows >= every ksl[r + 1] - ksl[r]; kp (S,) int32 gets their positions. cos_t / sin_t NULL: keys as
+ * stored. Rows outside the pools (epool_elems, sink_elems bf16 elements) are zeros; sources need no alignment; k / v may be NULL
+ * when no row has new rows. */
+int kv800_hip_window_keys(const kv800_paged_t* P, int64_t R, int64_t max_rows, const uint16_t* cos_t,
+                          const uint16_t* sin_t, int64_t rope_rows, int64_t epool_elems, int64_t sink_elems,
+                          int64_t nsink, const int64_t* prev, const int64_t* qsl, const int64_t* ksl, const uint16_t* k,
+                          const uint16_t* v, uint16_t* k_out, uint16_t* v_out, int32_t* kp, void* stream);
+
 /* Keys (S, 4, 128) bf16 rotated at positions pos (S,) int64 with the (rope_rows, 32) bf16 tables of the 32 rotating
  * frequencies, replacing the reference's _rope over its 128-wide tables (vllm_attn.py:160-163): per element
  * k * c + rot(k) * s in fp32 with c = 1, s = 0 on dims without a frequency, rounded to bf16 -- bit-identical. out may

@@ -862,14 +862,61 @@ __device__ __forceinline__ uint4 pack_bf16x8(const float (&x)[8]) {
 
 // positions per history workgroup
 constexpr int HPOS = 32, HPOS_MIN = 16, HPOS_MIN_GROUPS = 1024;
+// The new rows of a prefill chunk, appended to each row's history by the workgroups after its `tiles` history tiles
+// (the copy and rotation of rope_rows_kernel; one launch where the history, the rotation and two index copies took four).
+struct NewRows {
+  const uint16_t* k;      // (T, 4, 128) new rows, row r's at [qsl[r], qsl[r + 1])
+  const uint16_t* v;
+  const int64_t* prev;    // history lengths (instead of P.N); null: history only
+  const int64_t* qsl;
+  int tiles;              // history tiles of the grid
+};
+constexpr int NEW_ROWS = 32;   // new rows per workgroup
+
+// One unit of a plain K / V row: dims d0 .. d0 + 7 and d0 + 64 .. of one head from kr / vr (any alignment) to ko / vo,
+// the keys rotated at position pos when cos_t is given (clamped into the tables)
+__device__ __forceinline__ void copy_unit(const uint16_t* kr, const uint16_t* vr, uint16_t* ko, uint16_t* vo, int d0,
+                                          int64_t pos, const uint16_t* cos_t, const uint16_t* sin_t, int64_t rope_rows) {
+  const uint4 k0 = load16(reinterpret_cast<const uint8_t*>(kr + d0)), k1 = load16(reinterpret_cast<const uint8_t*>(kr + d0 + 64));
+  *reinterpret_cast<uint4*>(vo + d0) = load16(reinterpret_cast<const uint8_t*>(vr + d0));
+  *reinterpret_cast<uint4*>(vo + d0 + 64) = load16(reinterpret_cast<const uint8_t*>(vr + d0 + 64));
+  if (!cos_t) {
+    *reinterpret_cast<uint4*>(ko + d0) = k0;
+    *reinterpret_cast<uint4*>(ko + d0 + 64) = k1;
+    return;
+  }
+  const uint32_t wa[4] = {k0.x, k0.y, k0.z, k0.w}, wb[4] = {k1.x, k1.y, k1.z, k1.w};
+  float a[8], b[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    a[e] = (e & 1) ? bf2f_hi(wa[e >> 1]) : bf2f_lo(wa[e >> 1]);
+    b[e] = (e & 1) ? bf2f_hi(wb[e >> 1]) : bf2f_lo(wb[e >> 1]);
+  }
+  pos = min(max(pos, (int64_t)0), rope_rows - 1);
+  rope8(a, b, cos_t + pos * 32 + d0, sin_t + pos * 32 + d0, d0 < 32);
+  *reinterpret_cast<uint4*>(ko + d0) = pack_bf16x8(a);
+  *reinterpret_cast<uint4*>(ko + d0 + 64) = pack_bf16x8(b);
+}
+
 __global__ void __launch_bounds__(256) history_kernel(kv800_paged_t P, const uint16_t* __restrict__ cos_t,
                                                       const uint16_t* __restrict__ sin_t, int64_t rope_rows,
                                                       int64_t qpool_bytes, int64_t epool_elems,
                                                       const int64_t* __restrict__ out_off, uint16_t* __restrict__ kout,
-                                                      uint16_t* __restrict__ vout, int hpos) {
+                                                      uint16_t* __restrict__ vout, int hpos, NewRows X) {
   __shared__ float klo_s[512], ksc_s[512];
   const int r = blockIdx.y, tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-  const int n = P.N[r], p0 = blockIdx.x * hpos;
+  const int n = X.prev ? (int)X.prev[r] : P.N[r];
+  if (X.prev && (int)blockIdx.x >= X.tiles) {
+    const int64_t q0 = X.qsl[r], i0 = (int64_t)((int)blockIdx.x - X.tiles) * NEW_ROWS;
+    const int cnt = (int)min((int64_t)NEW_ROWS, X.qsl[r + 1] - q0 - i0);
+    for (int u = tid; u < cnt * 32; u += 256) {
+      const int h = (u >> 3) & 3, d0 = 8 * (u & 7);
+      const int64_t i = i0 + (u >> 5), src = (q0 + i) * 512 + h * 128, dst = (out_off[r] + n + i) * 512 + h * 128;
+      copy_unit(X.k + src, X.v + src, kout + dst, vout + dst, d0, n + i, cos_t, sin_t, rope_rows);
+    }
+    return;
+  }
+  const int p0 = blockIdx.x * hpos;
   if (p0 >= n) return;   // uniform over the workgroup
   const int cnt = min(hpos, n - p0);
   const int sb = p0 / BLK, to = p0 - sb * BLK;   // the positions' sub-block and the first one's token in it
@@ -1008,6 +1055,55 @@ __global__ void __launch_bounds__(256) history_kernel(kv800_paged_t P, const uin
   }
 }
 
+// ---------------------------------------------------------------- prefill keys of a window layer
+// Row r's attended rows in order, (its sinks, its kept exact rows [lo, prev), its new rows), as contiguous K (rotated at
+// their positions when cos_t is given) and V at output rows ksl[r] + i, with their positions in kp: one launch for what
+// the host assembled with some 40 gathers, concatenations and index uploads. lo = max(0, prev - (win - 1)), sinks
+// 0 .. min(nsink, lo) - 1. Rows outside the pools are zeros. A workgroup copies WIN_ROWS rows, 32 units a row.
+// 8 rows of 2,048 new tokens over a full window: the whole call 555 -> 134 us.
+constexpr int WIN_ROWS = 32;
+__global__ void __launch_bounds__(256) window_keys_kernel(kv800_paged_t P, const uint16_t* __restrict__ cos_t,
+                                                          const uint16_t* __restrict__ sin_t, int64_t rope_rows,
+                                                          int64_t epool_elems, int64_t sink_elems, int nsink,
+                                                          const int64_t* __restrict__ prev, const int64_t* __restrict__ ksl,
+                                                          const int64_t* __restrict__ qsl,
+                                                          const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
+                                                          uint16_t* __restrict__ kout, uint16_t* __restrict__ vout,
+                                                          int32_t* __restrict__ kp) {
+  const int r = blockIdx.y;
+  const int64_t n = prev[r], lo = max(n - (P.win - 1), (int64_t)0), ns = min((int64_t)nsink, lo);
+  const int64_t rows = ksl[r + 1] - ksl[r], i0 = (int64_t)blockIdx.x * WIN_ROWS;
+  const int cnt = (int)min((int64_t)WIN_ROWS, rows - i0);
+  for (int u = threadIdx.x; u < cnt * 32; u += 256) {
+    const int h = (u >> 3) & 3, d0 = 8 * (u & 7);
+    const int64_t i = i0 + (u >> 5), dst = (ksl[r] + i) * 512 + h * 128;
+    const int64_t pos = i < ns ? i : lo + (i - ns);
+    const uint16_t *kr = nullptr, *vr = nullptr;
+    if (i < ns) {
+      const int64_t a = P.skoff[r] + (i * 4 + h) * 128, b = P.svoff[r] + (i * 4 + h) * 128;
+      if (a >= 0 && b >= 0 && a + 128 <= sink_elems && b + 128 <= sink_elems) { kr = P.sk + a; vr = P.sv + b; }
+    } else if (pos < n) {
+      const int64_t pg = pos / P.ebs, base = pg < P.eoff_stride ? P.eoff[r * P.eoff_stride + pg] : -1;
+      const int64_t a = base + h * P.e_hs + (pos - pg * P.ebs) * P.e_ts, b = a + P.e_v;
+      if (base >= 0 && a >= 0 && b >= 0 && a + 128 <= epool_elems && b + 128 <= epool_elems) {
+        kr = P.epool + a;
+        vr = P.epool + b;
+      }
+    } else {
+      kr = k + (qsl[r] + (pos - n)) * 512 + h * 128;
+      vr = v + (qsl[r] + (pos - n)) * 512 + h * 128;
+    }
+    if ((u & 31) == 0) kp[ksl[r] + i] = (int32_t)pos;
+    if (kr) {
+      copy_unit(kr, vr, kout + dst, vout + dst, d0, pos, cos_t, sin_t, rope_rows);
+    } else {
+      const uint4 zero4 = make_uint4(0, 0, 0, 0);
+      *reinterpret_cast<uint4*>(kout + dst + d0) = zero4; *reinterpret_cast<uint4*>(kout + dst + d0 + 64) = zero4;
+      *reinterpret_cast<uint4*>(vout + dst + d0) = zero4; *reinterpret_cast<uint4*>(vout + dst + d0 + 64) = zero4;
+    }
+  }
+}
+
 }  // namespace
 }  // namespace kv800
 
@@ -1103,13 +1199,10 @@ int kv800_hip_fake_quant_v(const float* v, int64_t N, float* out, void* stream) 
   return check_launch("fake_quant_v");
 }
 
-int kv800_hip_history(const kv800_paged_t* P, int64_t R, int64_t max_n, const uint16_t* cos_t, const uint16_t* sin_t,
-                       int64_t rope_rows, int64_t qpool_bytes, int64_t epool_elems, const int64_t* out_off,
-                       uint16_t* k_out, uint16_t* v_out, void* stream) {
-  g_err[0] = 0;
-  KV800_REQUIRE(P && R >= 0 && max_n >= 0, "history: bad arguments");
-  if (R == 0 || max_n == 0) return KV800_OK;
-  KV800_REQUIRE(P->N && P->NQ && P->epool && P->eoff && out_off && k_out && v_out, "history: null pointer");
+// The history launch, with the chunk's new rows when X.k is given (max_new their largest count per row).
+static int launch_history(const kv800_paged_t* P, int64_t R, int64_t max_n, const uint16_t* cos_t, const uint16_t* sin_t,
+                          int64_t rope_rows, int64_t qpool_bytes, int64_t epool_elems, const int64_t* out_off,
+                          uint16_t* k_out, uint16_t* v_out, NewRows X, int64_t max_new, void* stream) {
   KV800_REQUIRE(!cos_t == !sin_t, "history: cos_t and sin_t go together");
   KV800_REQUIRE(P->ebs > 0 && P->e_hs % 8 == 0 && P->e_ts % 8 == 0 && P->e_v % 8 == 0 && ((uintptr_t)P->epool % 16) == 0,
                 "history: exact strides must be multiples of 8 elements and the pool 16-byte aligned");
@@ -1118,11 +1211,57 @@ int kv800_hip_history(const kv800_paged_t* P, int64_t R, int64_t max_n, const ui
   KV800_REQUIRE(R <= 65535, "history: at most 65535 rows per call");
   int hpos = HPOS;
   while (hpos > HPOS_MIN && (max_n + hpos - 1) / hpos * R < HPOS_MIN_GROUPS) hpos /= 2;
-  const int64_t tiles = (max_n + hpos - 1) / hpos;
-  KV800_REQUIRE(tiles <= 0x7FFFFFFF, "history: max_n too large");
-  hipLaunchKernelGGL(history_kernel, dim3((unsigned)tiles, (unsigned)R), dim3(256), 0, (hipStream_t)stream, *P, cos_t,
-                     sin_t, rope_rows, qpool_bytes, epool_elems, out_off, k_out, v_out, hpos);
+  const int64_t tiles = (max_n + hpos - 1) / hpos, grid = tiles + (max_new + NEW_ROWS - 1) / NEW_ROWS;
+  KV800_REQUIRE(grid <= 0x7FFFFFFF, "history: max_n too large");
+  X.tiles = (int)tiles;
+  hipLaunchKernelGGL(history_kernel, dim3((unsigned)grid, (unsigned)R), dim3(256), 0, (hipStream_t)stream, *P, cos_t,
+                     sin_t, rope_rows, qpool_bytes, epool_elems, out_off, k_out, v_out, hpos, X);
   return check_launch("history");
+}
+
+int kv800_hip_history(const kv800_paged_t* P, int64_t R, int64_t max_n, const uint16_t* cos_t, const uint16_t* sin_t,
+                       int64_t rope_rows, int64_t qpool_bytes, int64_t epool_elems, const int64_t* out_off,
+                       uint16_t* k_out, uint16_t* v_out, void* stream) {
+  g_err[0] = 0;
+  KV800_REQUIRE(P && R >= 0 && max_n >= 0, "history: bad arguments");
+  if (R == 0 || max_n == 0) return KV800_OK;
+  KV800_REQUIRE(P->N && P->NQ && P->epool && P->eoff && out_off && k_out && v_out, "history: null pointer");
+  return launch_history(P, R, max_n, cos_t, sin_t, rope_rows, qpool_bytes, epool_elems, out_off, k_out, v_out, NewRows{},
+                        0, stream);
+}
+
+int kv800_hip_prefill_keys(const kv800_paged_t* P, int64_t R, int64_t max_prev, int64_t max_new, const uint16_t* cos_t,
+                           const uint16_t* sin_t, int64_t rope_rows, int64_t qpool_bytes, int64_t epool_elems,
+                           const int64_t* prev, const int64_t* qsl, const int64_t* ksl, const uint16_t* k,
+                           const uint16_t* v, uint16_t* k_out, uint16_t* v_out, void* stream) {
+  g_err[0] = 0;
+  KV800_REQUIRE(P && R >= 0 && max_prev >= 0 && max_new >= 0, "prefill_keys: bad arguments");
+  if (R == 0 || max_prev + max_new == 0) return KV800_OK;
+  KV800_REQUIRE(P->NQ && P->epool && P->eoff && prev && qsl && ksl && (!max_new || (k && v)) && k_out && v_out,
+                "prefill_keys: null pointer");
+  KV800_REQUIRE(!cos_t || rope_rows > 0, "prefill_keys: empty RoPE tables");
+  return launch_history(P, R, max_prev, cos_t, sin_t, rope_rows, qpool_bytes, epool_elems, ksl, k_out, v_out,
+                        NewRows{k, v, prev, qsl, 0}, max_new, stream);
+}
+
+int kv800_hip_window_keys(const kv800_paged_t* P, int64_t R, int64_t max_rows, const uint16_t* cos_t,
+                          const uint16_t* sin_t, int64_t rope_rows, int64_t epool_elems, int64_t sink_elems,
+                          int64_t nsink, const int64_t* prev, const int64_t* qsl, const int64_t* ksl, const uint16_t* k,
+                          const uint16_t* v, uint16_t* k_out, uint16_t* v_out, int32_t* kp, void* stream) {
+  g_err[0] = 0;
+  KV800_REQUIRE(P && R >= 0 && max_rows >= 0 && nsink >= 0, "window_keys: bad arguments");
+  if (R == 0 || max_rows == 0) return KV800_OK;
+  KV800_REQUIRE(P->epool && P->eoff && prev && qsl && ksl && k_out && v_out && kp, "window_keys: null pointer");
+  KV800_REQUIRE(!nsink || (P->sk && P->sv && P->skoff && P->svoff), "window_keys: sinks need sk, sv, skoff and svoff");
+  KV800_REQUIRE(!cos_t == !sin_t && (!cos_t || rope_rows > 0), "window_keys: cos_t and sin_t go together, with rows");
+  KV800_REQUIRE(P->ebs > 0 && P->win > 0, "window_keys: ebs and win must be > 0");
+  KV800_REQUIRE(((uintptr_t)k_out % 16) == 0 && ((uintptr_t)v_out % 16) == 0,
+                "window_keys: outputs must be 16-byte aligned");
+  KV800_REQUIRE(R <= 65535 && max_rows < (1ll << 31), "window_keys: at most 65535 rows of 2^31 keys per call");
+  hipLaunchKernelGGL(window_keys_kernel, dim3((unsigned)((max_rows + WIN_ROWS - 1) / WIN_ROWS), (unsigned)R), dim3(256), 0,
+                     (hipStream_t)stream, *P, cos_t, sin_t, rope_rows, epool_elems, sink_elems, (int)nsink, prev, ksl,
+                     qsl, k, v, k_out, v_out, kp);
+  return check_launch("window_keys");
 }
 
 }  // extern "C"

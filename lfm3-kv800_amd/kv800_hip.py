@@ -69,6 +69,10 @@ SIGNATURES = {
     "kv800_hip_page_offsets": (_I32, [_VP, _I64, _I64, _I64, _I64, _I64, _VP, _VP]),
     "kv800_hip_step_meta": (_I32, [_VP, _I64, _I64, _VP, _I64, _I64, _VP, _VP, _VP, _VP]),
     "kv800_hip_history": (_I32, [ctypes.POINTER(Paged), _I64, _I64, _VP, _VP, _I64, _I64, _I64, _VP, _VP, _VP, _VP]),
+    "kv800_hip_prefill_keys": (_I32, [ctypes.POINTER(Paged), _I64, _I64, _I64, _VP, _VP, _I64, _I64, _I64, _VP, _VP, _VP,
+                                      _VP, _VP, _VP, _VP, _VP]),
+    "kv800_hip_window_keys": (_I32, [ctypes.POINTER(Paged), _I64, _I64, _VP, _VP, _I64, _I64, _I64, _I64, _VP, _VP, _VP,
+                                     _VP, _VP, _VP, _VP, _VP, _VP]),
     "kv800_hip_rope_rows": (_I32, [_VP, _VP, _I64, _VP, _VP, _I64, _VP, _VP]),
     "kv800_hip_prefill": (_I32, [_VP, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _I64, _I64, _I64, _I64, _VP, _VP]),
     "kv800_hip_prefill_split": (_I32, [_VP, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _I64, _I64, _I64, _I64, _I64, _I64,
@@ -336,26 +340,11 @@ def history(P, lens, cos_t=None, sin_t=None, out=None, offs=None):
         return K, V, offs
     rot = cos_t is not None
     if rot:
-        _need(cos_t, "cos_t", torch.bfloat16, dev); _need(sin_t, "sin_t", torch.bfloat16, dev)
-        if cos_t.shape != sin_t.shape or cos_t.dim() != 2 or cos_t.shape[1] != 32:
-            raise ValueError("cos_t / sin_t must be (P, 32)")
-        cos_t, sin_t = cos_t.contiguous(), sin_t.contiguous()
-    _need(P.epool, "epool", torch.bfloat16, dev); _need(P.eoff, "eoff", torch.int64, dev)
-    _need(P.NQ, "NQ", torch.int32, dev)
-    if P.eoff.stride(-1) != 1 or P.eoff.shape[0] < R or P.NQ.shape[0] < R:
-        raise ValueError("eoff / NQ must cover the rows with contiguous eoff rows")
-    s = Paged()
-    s.epool, s.eoff, s.eoff_stride = P.epool.data_ptr(), P.eoff.data_ptr(), P.eoff.stride(0)
-    s.ebs, s.e_hs, s.e_ts, s.e_v = int(P.ebs), int(P.e_hs), int(P.e_ts), int(P.e_v)
+        cos_t, sin_t = _rope32(cos_t, sin_t, dev)
+    s = _exact_struct(P, R)
+    qbytes = _quant_struct(s, P, R, dev)
     N = host_to_device(lens, torch.int32, dev)   # the output extents, from the host lengths
-    s.N, s.NQ = N.data_ptr(), P.NQ.data_ptr()
-    qbytes = 0
-    if P.qpool is not None and P.boff is not None and P.boff.numel():
-        _need(P.qpool, "qpool", torch.uint8, dev); _need(P.boff, "boff", torch.int64, dev)
-        if P.boff.stride(-1) != 1 or P.boff.shape[0] < R:
-            raise ValueError("boff must cover the rows with contiguous rows")
-        s.qpool, s.boff, s.boff_stride = P.qpool.data_ptr(), P.boff.data_ptr(), P.boff.stride(0)
-        qbytes = _extent(P.qpool)
+    s.N = N.data_ptr()
     offt = host_to_device(offs, torch.int64, dev)
     _check(L.kv800_hip_history(ctypes.byref(s), R, max(lens), _ptr(cos_t) if rot else None,
                                _ptr(sin_t) if rot else None, cos_t.shape[0] if rot else 0, qbytes, _extent(P.epool),
@@ -395,6 +384,30 @@ def prefill_splits(tiles, max_key_tiles):
     return int(max(1, min(64, -(-PREFILL_SPLIT_TARGET // w), max_key_tiles // 2)))
 
 
+class PrefillRows:
+    """Row geometry of a prefill call, on the host and (one upload) on the device: row r's queries / new rows
+    [qsl[r], qsl[r + 1]) from position qpos0[r] on, its keys [ksl[r], ksl[r + 1]), and the prefix sums of its 32-query
+    tiles."""
+
+    def __init__(self, qsl, ksl, qpos0, dev):
+        qsl, ksl, qpos0 = [int(x) for x in qsl], [int(x) for x in ksl], [int(x) for x in qpos0]
+        R = self.R = len(qpos0)
+        if len(qsl) != R + 1 or len(ksl) != R + 1:
+            raise ValueError("qsl and ksl need R + 1 entries")
+        tiles = [0]
+        for a, b in zip(qsl, qsl[1:]):
+            tiles.append(tiles[-1] + (b - a + 31) // 32)   # 32-query tiles, one workgroup per tile and KV head
+        self.qsl, self.ksl, self.qpos0, self.ntiles, self.dev = qsl, ksl, qpos0, tiles[-1], dev
+        self._host, self._meta = qsl + ksl + qpos0 + tiles, None
+
+    def ptrs(self):
+        """Device pointers of (qsl, ksl, qpos0, tiles); the tensor behind them lives as long as this object."""
+        if self._meta is None:
+            self._meta = host_to_device(self._host, torch.int64, self.dev)
+        p, n = self._meta.data_ptr(), self.R + 1
+        return tuple(ctypes.c_void_p(p + 8 * i) for i in (0, n, 2 * n, 3 * n - 1))
+
+
 def prefill(q, qsl, qpos0, K, V, kp, ksl, window=0, nsink=0, splits=None):
     """Prefill attention of ragged rows (kv800_hip_prefill_split): row r's queries q[qsl[r]:qsl[r+1]] ((T, 16, 128)
     bf16) at positions qpos0[r], qpos0[r] + 1, ... over keys / values K, V[ksl[r]:ksl[r+1]] ((S, 4, 128) bf16) at
@@ -402,14 +415,16 @@ def prefill(q, qsl, qpos0, K, V, kp, ksl, window=0, nsink=0, splits=None):
     (R + 1, R + 1, R). Mask: kp <= query
     position, and with window > 0 also kp > position - window or kp < nsink. splits: key splits per (query tile, KV
     head) (default prefill_splits: few query tiles over long rows are split and merged). Returns (T, 16, 128) bf16."""
+    return prefill_rows(q, PrefillRows(qsl, ksl, qpos0, q.device), K, V, kp, window, nsink, splits)
+
+
+def prefill_rows(q, rows, K, V, kp, window=0, nsink=0, splits=None):
+    """prefill with the row geometry already in a PrefillRows."""
     L = ops()
     dev = q.device
     q, K, V = q.contiguous(), K.contiguous(), V.contiguous()
     _need(q, "q", torch.bfloat16, dev); _need(K, "K", torch.bfloat16, dev); _need(V, "V", torch.bfloat16, dev)
-    qsl, ksl, qpos0 = [int(x) for x in qsl], [int(x) for x in ksl], [int(x) for x in qpos0]
-    R = len(qpos0)
-    if len(qsl) != R + 1 or len(ksl) != R + 1:
-        raise ValueError("qsl and ksl need R + 1 entries")
+    qsl, ksl, R = rows.qsl, rows.ksl, rows.R
     if q.dim() != 3 or q.shape[1:] != (16, 128) or qsl[0] != 0 or qsl[-1] != q.shape[0]:
         raise ValueError(f"q must be (qsl[-1], 16, 128), got {tuple(q.shape)}")
     if K.shape != V.shape or K.dim() != 3 or K.shape[1:] != (4, 128) or ksl[0] != 0 or ksl[-1] != K.shape[0]:
@@ -421,23 +436,130 @@ def prefill(q, qsl, qpos0, K, V, kp, ksl, window=0, nsink=0, splits=None):
         if kp.shape != (K.shape[0],):
             raise ValueError("kp must be (S,)")
     out = torch.empty(q.shape, dtype=torch.bfloat16, device=dev)
-    tiles = [0]
-    for a, b in zip(qsl, qsl[1:]):
-        tiles.append(tiles[-1] + (b - a + 31) // 32)   # 32-query tiles, one workgroup per tile and KV head
-    if R == 0 or tiles[-1] == 0:
+    if R == 0 or rows.ntiles == 0:
         return out
     if splits is None:
-        splits = prefill_splits(tiles[-1], max(-(-(b - a) // 64) for a, b in zip(ksl, ksl[1:])))
+        splits = prefill_splits(rows.ntiles, max(-(-(b - a) // 64) for a, b in zip(ksl, ksl[1:])))
     splits = int(splits)
     T = qsl[-1]
     part = torch.empty(T * 16 * splits * 132 if splits > 1 else 0, dtype=torch.float32, device=dev)
-    meta = host_to_device(qsl + ksl + qpos0 + tiles, torch.int64, dev)
-    m_qsl, m_ksl = meta[:R + 1], meta[R + 1:2 * R + 2]
-    m_pos, m_tiles = meta[2 * R + 2:3 * R + 2], meta[3 * R + 2:]
-    _check(L.kv800_hip_prefill_split(_ptr(q), _ptr(m_qsl), _ptr(m_pos), _ptr(K), _ptr(V), _ptr(kp), _ptr(m_ksl),
-                                     _ptr(m_tiles), R, tiles[-1], T, int(window), int(nsink), splits,
-                                     _ptr(part) if splits > 1 else None, part.numel(), _ptr(out), _stream(dev)))
+    m_qsl, m_ksl, m_pos, m_tiles = rows.ptrs()
+    _check(L.kv800_hip_prefill_split(_ptr(q), m_qsl, m_pos, _ptr(K), _ptr(V), _ptr(kp), m_ksl, m_tiles, R, rows.ntiles, T,
+                                     int(window), int(nsink), splits, _ptr(part) if splits > 1 else None, part.numel(),
+                                     _ptr(out), _stream(dev)))
     return out
+
+
+def _new_rows(k, v, T, dev):
+    """The chunk's new K / V rows as contiguous (T, 4, 128) bf16."""
+    k, v = k[:T].to(torch.bfloat16).contiguous(), v[:T].to(torch.bfloat16).contiguous()
+    _need(k, "k", torch.bfloat16, dev); _need(v, "v", torch.bfloat16, dev)
+    if k.shape != (T, 4, 128) or v.shape != (T, 4, 128):
+        raise ValueError(f"k / v must hold {T} rows (4, 128), got {tuple(k.shape)}, {tuple(v.shape)}")
+    return k, v
+
+
+def _rope32(cos_t, sin_t, dev):
+    _need(cos_t, "cos_t", torch.bfloat16, dev); _need(sin_t, "sin_t", torch.bfloat16, dev)
+    if cos_t.shape != sin_t.shape or cos_t.dim() != 2 or cos_t.shape[1] != 32:
+        raise ValueError("cos_t / sin_t must be (P, 32)")
+    return cos_t.contiguous(), sin_t.contiguous()
+
+
+def _exact_struct(P, R):
+    """kv800_paged_t with the exact pages of the first R rows of P."""
+    dev = P.epool.device
+    _need(P.epool, "epool", torch.bfloat16, dev); _need(P.eoff, "eoff", torch.int64, dev)
+    if P.eoff.stride(-1) != 1 or P.eoff.shape[0] < R:
+        raise ValueError("eoff must cover the rows with contiguous rows")
+    s = Paged()
+    s.epool, s.eoff, s.eoff_stride = P.epool.data_ptr(), P.eoff.data_ptr(), P.eoff.stride(0)
+    s.ebs, s.e_hs, s.e_ts, s.e_v = int(P.ebs), int(P.e_hs), int(P.e_ts), int(P.e_v)
+    return s
+
+
+def _quant_struct(s, P, R, dev):
+    """The quantized side of history rows into s; returns the quant pool's bytes."""
+    _need(P.NQ, "NQ", torch.int32, dev)
+    if P.NQ.shape[0] < R:
+        raise ValueError("NQ must cover the rows")
+    s.NQ = P.NQ.data_ptr()
+    if P.qpool is None or P.boff is None or not P.boff.numel():
+        return 0
+    _need(P.qpool, "qpool", torch.uint8, dev); _need(P.boff, "boff", torch.int64, dev)
+    if P.boff.stride(-1) != 1 or P.boff.shape[0] < R:
+        raise ValueError("boff must cover the rows with contiguous rows")
+    s.qpool, s.boff, s.boff_stride = P.qpool.data_ptr(), P.boff.data_ptr(), P.boff.stride(0)
+    return _extent(P.qpool)
+
+
+def prefill_keys(P, rows, k, v, cos_t, sin_t):
+    """All keys and values of a quantized layer's prefill rows, (S, 4, 128) bf16 each, in one launch
+    (kv800_hip_prefill_keys): per row of `rows` (a PrefillRows) its qpos0[r] history positions out of the cache P, then
+    its new rows of k / v, rotated."""
+    L = ops()
+    dev = P.epool.device
+    R, prev = rows.R, rows.qpos0
+    if any(x < 0 for x in prev):
+        raise ValueError("history lengths must be >= 0")
+    k, v = _new_rows(k, v, rows.qsl[-1], dev)
+    cos_t, sin_t = _rope32(cos_t, sin_t, dev)
+    K = torch.empty(rows.ksl[-1], 4, 128, dtype=torch.bfloat16, device=dev)
+    V = torch.empty_like(K)
+    if not R or not rows.ksl[-1]:
+        return K, V
+    if max(prev):
+        s = _exact_struct(P, R)
+        qbytes, eelems = _quant_struct(s, P, R, dev), _extent(P.epool)
+    else:                                    # no history: nothing of the cache is read
+        s, qbytes, eelems = Paged(), 0, 0
+        s.epool = s.eoff = s.NQ = K.data_ptr()
+        s.ebs = 1
+    m_qsl, m_ksl, m_pos, _ = rows.ptrs()
+    _check(L.kv800_hip_prefill_keys(ctypes.byref(s), R, max(prev), max(b - a for a, b in zip(rows.qsl, rows.qsl[1:])),
+                                    _ptr(cos_t), _ptr(sin_t), cos_t.shape[0], qbytes, eelems, m_pos, m_qsl, m_ksl,
+                                    _ptr(k), _ptr(v), _ptr(K), _ptr(V), _stream(dev)))
+    return K, V
+
+
+def window_keys(P, rows, k, v, cos_t, sin_t, win, nsink):
+    """The same for a window layer (kv800_hip_window_keys): sinks, kept exact rows, new rows; returns (K, V, positions
+    (S,) int32). cos_t None: keys as stored."""
+    L = ops()
+    dev = P.epool.device
+    R = rows.R
+    k, v = _new_rows(k, v, rows.qsl[-1], dev)
+    if cos_t is not None:
+        cos_t, sin_t = _rope32(cos_t, sin_t, dev)
+    K = torch.empty(rows.ksl[-1], 4, 128, dtype=torch.bfloat16, device=dev)
+    V = torch.empty_like(K)
+    kp = torch.empty(rows.ksl[-1], dtype=torch.int32, device=dev)
+    if not R or not rows.ksl[-1]:
+        return K, V, kp
+    eoff = P.eoff if P.eoff.stride(-1) == 1 else P.eoff.contiguous()
+    _need(P.epool, "epool", torch.bfloat16, dev); _need(eoff, "eoff", torch.int64, dev)
+    if eoff.shape[0] < R or any(n > 0 and (n - 1) // int(P.ebs) >= eoff.shape[1] for n in rows.qpos0):
+        raise IndexError("eoff does not cover the rows' positions")
+    s = Paged()
+    s.epool, s.eoff, s.eoff_stride = P.epool.data_ptr(), eoff.data_ptr(), eoff.stride(0)
+    s.ebs, s.e_hs, s.e_ts, s.e_v = int(P.ebs), int(P.e_hs), int(P.e_ts), int(P.e_v)
+    s.win = win
+    sink_elems = 0
+    if nsink:
+        _need(P.sk, "sk", torch.bfloat16, dev); _need(P.sv, "sv", torch.bfloat16, dev)
+        _need(P.skoff, "skoff", torch.int64, dev); _need(P.svoff, "svoff", torch.int64, dev)
+        skoff, svoff = P.skoff.contiguous(), P.svoff.contiguous()
+        if skoff.shape[0] < R or svoff.shape[0] < R:
+            raise IndexError("skoff / svoff must cover the rows")
+        s.sk, s.sv, s.skoff, s.svoff = P.sk.data_ptr(), P.sv.data_ptr(), skoff.data_ptr(), svoff.data_ptr()
+        sink_elems = min(_extent(P.sk), _extent(P.sv))
+    m_qsl, m_ksl, m_pos, _ = rows.ptrs()
+    rot = cos_t is not None
+    _check(L.kv800_hip_window_keys(ctypes.byref(s), R, max(b - a for a, b in zip(rows.ksl, rows.ksl[1:])),
+                                   _ptr(cos_t) if rot else None, _ptr(sin_t) if rot else None,
+                                   cos_t.shape[0] if rot else 0, _extent(P.epool), sink_elems, nsink, m_pos, m_qsl, m_ksl,
+                                   _ptr(k), _ptr(v), _ptr(K), _ptr(V), _ptr(kp), _stream(dev)))
+    return K, V, kp
 
 
 def read_probe(buf, out, groups):

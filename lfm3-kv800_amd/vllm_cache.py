@@ -384,39 +384,37 @@ def _ranges(starts, counts):
     return base + np.arange(int(counts.sum()), dtype=np.int64)
 
 
+def _rows(qsl, counts, prev, dev):
+    """PrefillRows of rows with `counts` keys before their new rows qsl[i] .. qsl[i + 1], from position prev[i] on."""
+    ksl = [0]
+    for i, c in enumerate(counts):
+        ksl.append(ksl[-1] + c + qsl[i + 1] - qsl[i])
+    return kv800_hip.PrefillRows(qsl, ksl, prev, dev)
+
+
 def prefill_quant_rows(P, q, k, v, qsl, prev, cos_t, sin_t):
     """Prefill / extend rows of a quantized layer (vllm_attn.py:351-402 for quant layers): row i has queries
     q[qsl[i]:qsl[i+1]] (post-RoPE) at positions prev[i] .. prev[i] + (qsl[i+1] - qsl[i]) - 1, new pre-RoPE keys and
     values k / v at the same rows, and a history of prev[i] positions in the cache P (its first (prev - 128) // 256
-    sub-blocks flushed, P.NQ, the rest in the exact pages). The history comes out of one kv800_hip_history launch
-    (dequantized, rotated, bf16), the new keys out of one kv800_hip_rope_rows launch; each row's keys are its history
-    followed by its new rows, and one kv800_hip_prefill launch attends all rows. qsl / prev are host sequences.
-    Returns (T, 16, 128) bf16."""
-    return kv800_hip.prefill(*prefill_quant_inputs(P, q, k, v, qsl, prev, cos_t, sin_t), window=0)
+    sub-blocks flushed, P.NQ, the rest in the exact pages). One kv800_hip_prefill_keys launch writes each row's history
+    (dequantized, rotated, bf16) followed by its new rows (rotated), and one kv800_hip_prefill launch attends all rows.
+    qsl / prev are host sequences. Returns (T, 16, 128) bf16."""
+    rows, K, V = _quant_rows(P, q, k, v, qsl, prev, cos_t, sin_t)
+    return kv800_hip.prefill_rows(q, rows, K, V, None)
+
+
+def _quant_rows(P, q, k, v, qsl, prev, cos_t, sin_t):
+    prev, qsl = [int(x) for x in prev], [int(x) for x in qsl]
+    rows = _rows(qsl, prev, prev, q.device)
+    return rows, *kv800_hip.prefill_keys(P, rows, k, v, cos_t, sin_t)
 
 
 def prefill_quant_inputs(P, q, k, v, qsl, prev, cos_t, sin_t):
     """The arguments of prefill_quant_rows' attention launch, (q, qsl, prev, K, V, key positions, key row starts):
     the rows' keys (history, then new rows) and values assembled as prefill_quant_rows describes. The key positions
     are None: key j of a row is at position j."""
-    dev = q.device
-    prev, qsl = [int(x) for x in prev], [int(x) for x in qsl]
-    new = [b - a for a, b in zip(qsl, qsl[1:])]
-    T = qsl[-1]
-    # key order: row 0's history, row 0's new rows, row 1's history, ...; the history launch writes each row's history
-    # in place, the new rows (rotated) follow by one index_copy_ each for K and V
-    ksl = np.concatenate(([0], np.cumsum(np.asarray(prev) + np.asarray(new)))).astype(np.int64)
-    Kc = torch.empty(int(ksl[-1]), 4, 128, dtype=torch.bfloat16, device=dev)
-    Vc = torch.empty_like(Kc)
-    kv800_hip.history(P, prev, cos_t, sin_t, out=(Kc, Vc), offs=ksl[:-1])
-    # the new rows' positions and their key indices, in one copy
-    pi = kv800_hip.host_to_device(np.concatenate((_ranges(prev, new), _ranges(ksl[:-1] + np.asarray(prev, np.int64),
-                                                                              new))), torch.int64, dev)
-    pos_new, idx = pi[:T], pi[T:]
-    Kn = kv800_hip.rope_rows(k[:T].to(torch.bfloat16), pos_new, cos_t, sin_t)
-    Kc.index_copy_(0, idx, Kn)
-    Vc.index_copy_(0, idx, v[:T].to(torch.bfloat16))
-    return q, qsl, prev, Kc, Vc, None, ksl   # key positions: the index within the row (kp = None)
+    rows, K, V = _quant_rows(P, q, k, v, qsl, prev, cos_t, sin_t)
+    return q, rows.qsl, rows.qpos0, K, V, None, np.asarray(rows.ksl, np.int64)
 
 
 def prefill_window_rows(P, q, k, v, qsl, prev, cos_t, sin_t):
@@ -426,50 +424,11 @@ def prefill_window_rows(P, q, k, v, qsl, prev, cos_t, sin_t):
     set) at P.skoff / P.svoff in P.sk / P.sv, and the exact rows [lo, prev[i]) with lo = max(0, prev[i] - (WIN - 1)) in
     the exact pages of P (P.eoff element offsets per ebs positions, e_hs / e_ts / e_v strides). With cos_t / sin_t all
     keys are rotated at their positions (window + sinks layers keep pre-RoPE keys); None leaves them as stored (sliding
-    layers keep post-RoPE keys). One gather of the history, then one kv800_hip_prefill launch with the window mask
-    (and the sinks). qsl / prev are host sequences. Returns (T, 16, 128) bf16."""
-    dev = q.device
+    layers keep post-RoPE keys). One kv800_hip_window_keys launch, then one kv800_hip_prefill launch with the window
+    mask (and the sinks). qsl / prev are host sequences. Returns (T, 16, 128) bf16."""
     prev, qsl = [int(x) for x in prev], [int(x) for x in qsl]
-    R = len(prev)
-    new = np.asarray([b - a for a, b in zip(qsl, qsl[1:])], np.int64)
-    p0 = np.asarray(prev, np.int64)
-    lo = np.maximum(0, p0 - (kv800.WIN - 1))
-    sinks = P.sk is not None
-    ns = np.minimum(kv800.NSINK, lo) if sinks else np.zeros(R, np.int64)
-    nx = p0 - lo
-    rows = np.arange(R)
-    # ---- exact rows [lo, prev): element offset of each (position, head) K row through the page table
-    xr = np.repeat(rows, nx)
-    xp = _ranges(lo, nx)
-    h2d = lambda a: kv800_hip.host_to_device(a, torch.int64, dev)
-    page = P.eoff[h2d(xr), h2d(xp // P.ebs)]                                      # (Sx,) element offsets
-    ko = (page + h2d((xp % P.ebs) * P.e_ts))[:, None] + torch.arange(4, device=dev) * P.e_hs
-    d128 = torch.arange(128, device=dev)
-    ef = kv800.flat(P.epool)
-    Kx, Vx = ef[ko[..., None] + d128], ef[ko[..., None] + P.e_v + d128]                          # (Sx, 4, 128)
-    # ---- sink rows
-    if sinks:
-        sr = np.repeat(rows, ns)
-        st = _ranges(np.zeros(R, np.int64), ns)
-        so = h2d(st * 512)[:, None] + torch.arange(4, device=dev) * 128
-        srd = h2d(sr)
-        Ks = kv800.flat(P.sk)[(P.skoff[srd][:, None] + so)[..., None] + d128]
-        Vs = kv800.flat(P.sv)[(P.svoff[srd][:, None] + so)[..., None] + d128]
-    else:
-        Ks = Vs = torch.empty(0, 4, 128, dtype=torch.bfloat16, device=dev)
-    # ---- per row: sinks, exact rows, new rows, as rows of cat(sinks, exact, new)
-    cnt = ns + nx + new
-    ksl = np.concatenate(([0], np.cumsum(cnt))).astype(np.int64)
-    order = np.concatenate([np.concatenate((_ranges([s0], [a]), len(Ks) + _ranges([x0], [b]),
-                                            len(Ks) + len(Kx) + _ranges([q0], [c])))
-                            for s0, x0, q0, a, b, c in zip(np.cumsum(ns) - ns, np.cumsum(nx) - nx, qsl[:-1], ns, nx,
-                                                           new)]) if R else np.zeros(0, np.int64)
-    kpos = np.concatenate([np.concatenate((np.arange(a), np.arange(l0, n0), np.arange(n0, n0 + c)))
-                           for a, l0, n0, c in zip(ns, lo, p0, new)]) if R else np.zeros(0, np.int64)
-    idx = h2d(order.astype(np.int64))
-    Kc = torch.cat((Ks, Kx, k[:qsl[-1]].to(torch.bfloat16))).index_select(0, idx)
-    Vc = torch.cat((Vs, Vx, v[:qsl[-1]].to(torch.bfloat16))).index_select(0, idx)
-    if cos_t is not None:
-        Kc = kv800_hip.rope_rows(Kc, h2d(kpos), cos_t, sin_t)
-    return kv800_hip.prefill(q, qsl, prev, Kc, Vc, torch.from_numpy(kpos.astype(np.int32)), ksl, window=kv800.WIN,
-                             nsink=kv800.NSINK if sinks else 0)
+    nsink = kv800.NSINK if P.sk is not None else 0
+    kept = [min(n, kv800.WIN - 1) + min(nsink, max(0, n - (kv800.WIN - 1))) for n in prev]
+    rows = _rows(qsl, kept, prev, q.device)
+    K, V, kp = kv800_hip.window_keys(P, rows, k, v, cos_t, sin_t, kv800.WIN, nsink)
+    return kv800_hip.prefill_rows(q, rows, K, V, kp, window=kv800.WIN, nsink=nsink)
