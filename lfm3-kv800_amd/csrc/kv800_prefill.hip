@@ -14,20 +14,23 @@
 //                     online softmax, bf16 probabilities for the P.V product, fp32 accumulation, bf16 out.
 //
 // prefill_kernel, one workgroup = 32 consecutive queries of one row and one KV head g; wave w computes query head
-// 4 g + w for its 32 queries as two 16-query blocks, so the 4 waves share each 64-key tile staged in LDS. Per wave and
-// tile, with v_mfma_f32_16x16x32_bf16 (lane l: D column l % 16, D rows 4 (l / 16) + 0..3; A row l % 16 and B column
-// l % 16 over k = 8 (l / 16) + 0..7):
+// 4 g + w for its 32 queries, so the 4 waves share each 64-key tile staged in LDS. Per wave and tile, with
+// v_mfma_f32_32x32x16_bf16 (lane l: D column l % 32, D rows 8 c + 4 (l / 32) + 0..3; A row l % 32 and B column l % 32
+// over k = 8 (l / 32) + 0..7):
 //   S^T = K . Q^T   (keys x queries): A = K rows from LDS, B = the wave's queries held in registers;
 //   O^T += V^T . P^T (dims x queries): A = V^T read from the V rows by ds_read_b64_tr_b16, B = the lane's own
-//                    probabilities;
-// each A operand feeds both query blocks. Both results keep one query per lane column (l % 16), so the softmax
-// statistics of a query live in the four lanes l % 16 and are combined with two cross-lane steps, and the O rescale
-// (lazy: only when a query's running max grows by more than PLAZY) needs no data movement. P^T's B operand is the
-// lane's 8 probabilities of keys 4 G + i and 16 + 4 G + i (G = l / 16) of each 32-key half, the key order in which
-// the transposed reads deliver V^T. The tiles are double-buffered in LDS and loaded straight into it (buffer loads
-// with the lds modifier, through a buffer resource whose reads past the row's keys return zeros; the next tile's
-// loads are in flight while the current one is multiplied, one barrier per tile), and a tile whose keys are all in
-// range and precede the workgroup's first query is not masked.
+//                    probabilities.
+// Both results keep one query per lane column (l % 32), so the softmax statistics of a query live in two lanes and are
+// combined with one cross-lane step, and the O rescale (lazy: only when a query's running max grows by more than PLAZY)
+// needs no data movement. P^T's B operand is the lane's 8 probabilities of keys 4 G + i and 8 + 4 G + i (G = l / 32) of
+// each 16-key step, the key order in which the transposed reads deliver V^T. The tiles are double-buffered in LDS and
+// loaded straight into it (buffer loads with the lds modifier, through a buffer resource whose reads past the row's keys
+// return zeros; the next tile's loads are in flight while the current one is multiplied, one barrier per tile), and a
+// tile whose keys are all in range and precede the workgroup's first query is not masked.
+// Bound: matrix and VALU issue, which overlap only in part, at the clock the part holds under them (1.9 GHz here). 32 x 32
+// MFMA instead of twice as many 16 x 16 ones, with half the cross-lane steps, and the phase priorities: 8 rows x 2048
+// queries over 16K keys, whole call, 2,424 -> 2,370 -> 2,240 us (this kernel about 1.03 PFLOP/s; a library product of
+// 8192^3 reaches 1.14 on the same card).
 // Key tiles outside [first key a query of the workgroup can see, last key not in its future] are skipped: for window
 // layers only the sink keys and the keys of the window are read.
 // The grid is one workgroup per (KV head, 32-query tile), numbered so that each XCD runs whole (KV head, row) runs of
@@ -46,8 +49,10 @@ typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
 typedef short s4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s4 lds_s4;
 
-__device__ __forceinline__ f4 mfma_bf(u4v a, u4v b, f4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8, a), __builtin_bit_cast(b8, b), c, 0, 0, 0);
+typedef __bf16 mb8 __attribute__((ext_vector_type(8)));
+typedef float f16v __attribute__((ext_vector_type(16)));
+__device__ __forceinline__ f16v mfma_bf(u4v a, u4v b, f16v c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(mb8, a), __builtin_bit_cast(mb8, b), c, 0, 0, 0);
 }
 
 // ---------------------------------------------------------------- RoPE of key rows
@@ -78,25 +83,20 @@ __device__ __forceinline__ uint32_t bfpk(float a, float b) {
 
 // ---------------------------------------------------------------- flash attention of ragged rows
 // A workgroup of 4 waves takes PQ = 32 consecutive queries of one row (one interface tile) and one KV head g; wave w
-// computes query head 4 g + w for its 32 queries as two column blocks of 16. Every workgroup of the grid has work (a
+// computes query head 4 g + w for its 32 queries. Every workgroup of the grid has work (a
 // grid whose idle workgroups sat at every other index put all the work on half the XCDs under round-robin dispatch),
 // and the workgroups of one (KV head, row) run on one XCD, in order, so the row's key tiles are read once into that
 // XCD's L2 for its 64 query tiles. Keys come in tiles of 64, loaded into LDS as K and V rows by LDS-direct loads (no
 // register staging) and double-buffered: the next tile's loads are in flight while the current one is multiplied, one
-// barrier per tile. Per
-// wave and tile on f32_16x16x32_bf16: S^T = K . Q^T (keys x queries: 4 key blocks x 2 query blocks x 4 k-steps, every
-// K operand read once for both query blocks) and O^T += V^T . P^T (8 dim blocks x 2 query blocks x 2 k-steps; the
-// V^T operand is read from the V rows by two ds_read_b64_tr_b16, in the key order of the lane's own probabilities,
-// once for both query blocks), so both results keep one query per lane column: a query's softmax statistics live in
-// four lanes (two cross-lane steps) and the O rescale moves no data. A tile whose keys all precede the workgroup's
-// first query (and are all in range) needs no mask: in a chunk over a long history, nearly every tile.
+// barrier per tile. A tile whose keys all precede the workgroup's first query (and are all in range) needs no mask: in a
+// chunk over a long history, nearly every tile.
 constexpr int PQ = 32;      // queries per workgroup = per interface tile (tile_off counts these)
 constexpr int PPART = 132;  // floats per key-split partial of (query, head): 128 dims of o, m, l, 2 of padding
 constexpr int PMAXSPLIT = 256;
 constexpr int PK = 64;      // keys per LDS tile
 
 // a tile as staged by LDS-direct loads: K and V rows of 256 bytes, unpadded, their 16-byte pieces permuted within
-// each row so that the operand reads spread over the banks: piece p of key row j at piece p ^ (j & 15) (K: 16 rows
+// each row so that the operand reads spread over the banks: piece p of key row j at piece p ^ (j & 15) (K: 32 rows
 // read at one piece per instruction) and p ^ 2 (j & 7) (V: 32-byte pairs of pieces, 4 rows per 16 lanes)
 struct alignas(16) PTile {
   uint16_t k[PK * 128];
@@ -131,19 +131,14 @@ __device__ __forceinline__ int64_t upper(const int32_t* a, int64_t n, int64_t x)
   return lo;
 }
 
-// max / sum over the lanes l, l ^ 16, l ^ 32, l ^ 48 without an LDS round trip: v_permlane16_swap and
-// v_permlane32_swap on two copies of x leave both 16-lane (32-lane) halves in every lane of a pair. All 64 lanes must
-// be active.
-__device__ __forceinline__ float max4rows(float x) {
-  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  x = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-  r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+// x's values of lanes l and l ^ 32 without an LDS round trip: v_permlane32_swap on two copies of x leaves both halves in
+// every lane. All 64 lanes must be active.
+__device__ __forceinline__ float max2halves(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
   return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
-__device__ __forceinline__ float sum4rows(float x) {
-  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  x = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-  r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+__device__ __forceinline__ float sum2halves(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
@@ -162,7 +157,7 @@ prefill_kernel(const uint16_t* __restrict__ q, const int64_t* __restrict__ qsl, 
   const int ntl = nb / (4 * splits);
   const int g = L / (ntl * splits), h = 4 * g + w;
   const int lr = L - g * ntl * splits, sp = lr % splits;
-  const int col = lane & 15, G = lane >> 4;
+  const int col = lane & 31, G = lane >> 5;   // query column; key / dim half
   // ---- row of this tile: last i with tile_off[i] <= t
   const int64_t t = lr / splits;
   int64_t lo = 0, hi = R;
@@ -188,25 +183,19 @@ prefill_kernel(const uint16_t* __restrict__ q, const int64_t* __restrict__ qsl, 
   const int n0 = (int)((sink_end + PK - 1) / PK), nt = n0 + (int)((kend - kbeg + PK - 1) / PK);
   // key split sp of `splits` takes tiles [i0, i1) of the nt (all of them without a split)
   const int per_sp = (nt + splits - 1) / splits, i0 = min(nt, sp * per_sp), i1 = min(nt, i0 + per_sp);
-  // ---- the wave's queries as the B operands of S^T = K . Q^T (query block cq, 4 k-steps of 32 dims)
-  bool qok[2];
-  int qpos[2];
-  u4v qb[2][4];
+  // ---- the wave's queries as the B operands of S^T = K . Q^T (8 k-steps of 16 dims)
+  const bool qok = col < nq;
+  const int qpos = (int)(p0 + col);
+  u4v qb[8];
 #pragma unroll
-  for (int cq = 0; cq < 2; ++cq) {
-    qok[cq] = 16 * cq + col < nq;
-    qpos[cq] = (int)(p0 + 16 * cq + col);
+  for (int s = 0; s < 8; ++s)
+    qb[s] = qok ? *reinterpret_cast<const u4v*>(q + ((q0 + col) * 16 + h) * 128 + 16 * s + 8 * G) : u4v{0, 0, 0, 0};
+  f16v o[4];   // dims 32 j + 8 (v / 4) + 4 G + v % 4 of query col
 #pragma unroll
-    for (int s = 0; s < 4; ++s)
-      qb[cq][s] = qok[cq] ? *reinterpret_cast<const u4v*>(q + ((q0 + 16 * cq + col) * 16 + h) * 128 + 32 * s + 8 * G)
-                          : u4v{0, 0, 0, 0};
-  }
-  f4 o[2][8];
+  for (int j = 0; j < 4; ++j)
 #pragma unroll
-  for (int cq = 0; cq < 2; ++cq)
-#pragma unroll
-    for (int j = 0; j < 8; ++j) o[cq][j] = f4{0.f, 0.f, 0.f, 0.f};
-  float m[2] = {-1e30f, -1e30f}, lsum[2] = {0.f, 0.f};
+    for (int v = 0; v < 16; ++v) o[j][v] = 0.f;
+  float m = -1e30f, lsum = 0.f;
 
   // ---- tile i's keys [k0, k0 + 64) clipped to r1: from the sink range, then from the main range
   auto range_of = [&](int i, int64_t& k0, int64_t& r1) {
@@ -247,91 +236,84 @@ prefill_kernel(const uint16_t* __restrict__ q, const int64_t* __restrict__ qsl, 
   __syncthreads();
   auto step = [&](int i, const PTile& T, PTile& Nx) {
     if (i + 1 < i1) fetch(i + 1, Nx);
-    // ---- S^T = K . Q^T: 4 blocks of 16 keys x 2 blocks of 16 queries
-    f4 sc[2][4];
+    // ---- S^T = K . Q^T: 2 blocks of 32 keys; score register v of block nb: key 32 nb + 8 (v / 4) + 4 G + v % 4
+    // wave priority by phase: of a SIMD's two waves the one in its softmax (2) or P.V (1) goes before one in QK (0)
+    __builtin_amdgcn_s_setprio(0);
+    f16v sc[2];
 #pragma unroll
-    for (int nb = 0; nb < 4; ++nb) {
-      f4 a0 = {0.f, 0.f, 0.f, 0.f}, a1 = {0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < 8; ++s) {
+      const int po = 8 * kswz(col, 2 * s + G);   // rows col and 32 + col alike
 #pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        const u4v a = *reinterpret_cast<const u4v*>(&T.k[(nb * 16 + col) * 128 + 8 * kswz(col, 4 * s + G)]);
-        a0 = mfma_bf(a, qb[0][s], a0);
-        a1 = mfma_bf(a, qb[1][s], a1);
+      for (int nb = 0; nb < 2; ++nb) {
+        const u4v a = *reinterpret_cast<const u4v*>(&T.k[(nb * 32 + col) * 128 + po]);
+        const f16v zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        sc[nb] = mfma_bf(a, qb[s], s == 0 ? zero : sc[nb]);
       }
-      sc[0][nb] = a0;
-      sc[1][nb] = a1;
     }
-    // ---- mask, scale, online softmax per query block (the lane's 16 keys: nb * 16 + 4 G + i). No mask when every key
-    // of the tile is in range and precedes the workgroup's first query (quantized layers: no window).
+    // ---- mask, scale, online softmax (the lane's 32 keys). No mask when every key of the tile is in range and precedes
+    // the workgroup's first query (quantized layers: no window).
     int64_t tk0, tr1;
     range_of(i, tk0, tr1);
     const bool full = window <= 0 && tk0 + PK <= tr1 && (int64_t)T.kp[PK - 1] <= p0;
-    uint32_t pb[2][4][2];   // bf16 probabilities, packed in key pairs
+    if (!full) {
+      const int wlo = window > 0 ? (int)max((int64_t)qpos - window, (int64_t)INT32_MIN) : INT32_MIN;
+      const int ns = window > 0 ? (int)nsink : 0;
 #pragma unroll
-    for (int cq = 0; cq < 2; ++cq) {
-      if (!full) {
-        const int wlo = window > 0 ? (int)max((int64_t)qpos[cq] - window, (int64_t)INT32_MIN) : INT32_MIN;
-        const int ns = window > 0 ? (int)nsink : 0;
+      for (int nb = 0; nb < 2; ++nb) {
 #pragma unroll
-        for (int nb = 0; nb < 4; ++nb) {
-#pragma unroll
-          for (int i2 = 0; i2 < 4; ++i2) {
-            const int kpos = T.kp[nb * 16 + 4 * G + i2];
-            const bool keep = qok[cq] & (kpos <= qpos[cq]) & ((kpos > wlo) | (kpos < ns));
-            sc[cq][nb][i2] = keep ? sc[cq][nb][i2] : -INFINITY;
-          }
+        for (int v = 0; v < 16; ++v) {
+          const int kpos = T.kp[nb * 32 + 8 * (v >> 2) + 4 * G + (v & 3)];
+          const bool keep = qok & (kpos <= qpos) & ((kpos > wlo) | (kpos < ns));
+          sc[nb][v] = keep ? sc[nb][v] : -INFINITY;
         }
       }
-      float tmax = -INFINITY;
-#pragma unroll
-      for (int nb = 0; nb < 4; ++nb)
-        tmax = fmaxf(tmax, fmaxf(fmaxf(sc[cq][nb][0], sc[cq][nb][1]), fmaxf(sc[cq][nb][2], sc[cq][nb][3])));
-      tmax = max4rows(tmax) * scale_log2;   // scale > 0: the max of the scaled scores
-      if (__any(tmax > m[cq] + PLAZY)) {   // rescale only when a query's max outgrows its state (wave-uniform)
-        const float mnew = fmaxf(m[cq], tmax);
-        const float alpha = __builtin_amdgcn_exp2f(m[cq] - mnew);
-        m[cq] = mnew;
-        lsum[cq] *= alpha;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) o[cq][j] *= alpha;
-      }
-      const float mnew = m[cq];
-      float psum = 0.f;
-#pragma unroll
-      for (int nb = 0; nb < 4; ++nb) {
-        float p[4];
-#pragma unroll
-        for (int i2 = 0; i2 < 4; ++i2) {
-          p[i2] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[cq][nb][i2], scale_log2, -mnew));   // masked: -inf -> 0
-          psum += p[i2];
-        }
-        pb[cq][nb][0] = bfpk(p[0], p[1]);
-        pb[cq][nb][1] = bfpk(p[2], p[3]);
-      }
-      lsum[cq] += psum;
     }
-    // ---- O^T += V^T . P^T: 2 halves of 32 keys x 8 blocks of 16 dims x 2 query blocks. A = V^T (row = dim; K = the
-    // half's keys 4 G .. 4 G + 3 and 16 + 4 G .. + 3, whose probabilities the lane holds) by two transposed reads
-    const int vrow = 4 * G + (col >> 2);
+    __builtin_amdgcn_s_setprio(2);
+    float tmax = -INFINITY;
 #pragma unroll
-    for (int hh = 0; hh < 2; ++hh) {
-      const u4v b0 = {pb[0][2 * hh][0], pb[0][2 * hh][1], pb[0][2 * hh + 1][0], pb[0][2 * hh + 1][1]};
-      const u4v b1 = {pb[1][2 * hh][0], pb[1][2 * hh][1], pb[1][2 * hh + 1][0], pb[1][2 * hh + 1][1]};
+    for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int vo = 8 * vswz(vrow, 2 * j + ((col >> 1) & 1)) + 4 * (col & 1);   // rows vrow and vrow + 16 alike
+      for (int v = 0; v < 16; v += 2) tmax = fmaxf(fmaxf(tmax, sc[nb][v]), sc[nb][v + 1]);
+    tmax = max2halves(tmax) * scale_log2;   // scale > 0: the max of the scaled scores
+    if (__any(tmax > m + PLAZY)) {   // rescale only when a query's max outgrows its state (wave-uniform)
+      const float mnew = fmaxf(m, tmax);
+      const float alpha = __builtin_amdgcn_exp2f(m - mnew);
+      m = mnew;
+      lsum *= alpha;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[j] *= alpha;
+    }
+    // ---- O^T += V^T . P^T: 4 steps of 16 keys x 4 blocks of 32 dims. B = the step's 8 own probabilities (keys 4 G ..
+    // 4 G + 3 and 8 + 4 G .. + 3), A = V^T (row = dim; the same keys) by two transposed reads: 16-lane group lane / 16
+    // reads the key rows' dims 16 ((lane / 16) % 2) .. + 15 of the block
+    const int n16 = lane & 15, vrow = 4 * G + (n16 >> 2), vpc = 2 * ((lane >> 4) & 1) + ((n16 >> 1) & 1);
+    __builtin_amdgcn_s_setprio(1);
+    float psum = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      const int nb = ks >> 1, v0 = 8 * (ks & 1);
+      float p[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[nb][v0 + e], scale_log2, -m));   // masked: -inf -> 0
+        psum += p[e];
+      }
+      const u4v b = {bfpk(p[0], p[1]), bfpk(p[2], p[3]), bfpk(p[4], p[5]), bfpk(p[6], p[7])};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int vo = 8 * vswz(vrow, 4 * j + vpc) + 4 * (n16 & 1);   // rows vrow and vrow + 8 alike
         const s4 t0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (lds_s4*)const_cast<uint16_t*>(&T.v[(32 * hh + vrow) * 128 + vo]));
+            (lds_s4*)const_cast<uint16_t*>(&T.v[(16 * ks + vrow) * 128 + vo]));
         const s4 t1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (lds_s4*)const_cast<uint16_t*>(&T.v[(32 * hh + vrow + 16) * 128 + vo]));
+            (lds_s4*)const_cast<uint16_t*>(&T.v[(16 * ks + vrow + 8) * 128 + vo]));
         const u4v a = {__builtin_bit_cast(uint32_t, __builtin_shufflevector(t0, t0, 0, 1)),
                        __builtin_bit_cast(uint32_t, __builtin_shufflevector(t0, t0, 2, 3)),
                        __builtin_bit_cast(uint32_t, __builtin_shufflevector(t1, t1, 0, 1)),
                        __builtin_bit_cast(uint32_t, __builtin_shufflevector(t1, t1, 2, 3))};
-        o[0][j] = mfma_bf(a, b0, o[0][j]);
-        o[1][j] = mfma_bf(a, b1, o[1][j]);
+        o[j] = mfma_bf(a, b, o[j]);
       }
     }
+    lsum += psum;
     // the next tile's positions into its buffer, whose last reads (tile i - 1) ended at the previous barrier; the
     // barrier waits for the tile's LDS-direct loads
     if (i + 1 < i1 && tid < PK) Nx.kp[tid] = skp;
@@ -341,27 +323,29 @@ prefill_kernel(const uint16_t* __restrict__ q, const int64_t* __restrict__ qsl, 
     step(i, tA, tB);
     if (i + 1 < i1) step(i + 1, tB, tA);
   }
-  // ---- normalise and write: lane holds dims 16 j + 4 G + 0..3 of query 16 cq + col. With a key split, the
-  // unnormalised partial (o, m, l) of (query, head, split) instead: PPART floats, o relative to 2^m
+  // ---- normalise and write: lane holds dims 32 j + 8 c + 4 G + 0..3 of query col. With a key split, the unnormalised
+  // partial (o, m, l) of (query, head, split) instead: PPART floats, o relative to 2^m
+  const float l = sum2halves(lsum);
+  if (!qok) return;
+  if (part) {
+    float* pp = part + (((q0 + col) * 16 + h) * splits + sp) * PPART;
 #pragma unroll
-  for (int cq = 0; cq < 2; ++cq) {
-    const float l = sum4rows(lsum[cq]);
-    if (!qok[cq]) continue;
-    if (part) {
-      float* pp = part + (((q0 + 16 * cq + col) * 16 + h) * splits + sp) * PPART;
+    for (int j = 0; j < 4; ++j)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) *reinterpret_cast<f4*>(pp + 16 * j + 4 * G) = o[cq][j];
-      if (G == 0) { pp[128] = m[cq]; pp[129] = l; }
-      continue;
-    }
-    const float inv = l > 0.f ? 1.0f / l : 0.f;
-    uint16_t* dst = out + ((q0 + 16 * cq + col) * 16 + h) * 128 + 4 * G;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const u2v v2 = {bfpk(o[cq][j][0] * inv, o[cq][j][1] * inv), bfpk(o[cq][j][2] * inv, o[cq][j][3] * inv)};
-      *reinterpret_cast<u2v*>(dst + 16 * j) = v2;
-    }
+      for (int c = 0; c < 4; ++c)
+        *reinterpret_cast<f4*>(pp + 32 * j + 8 * c + 4 * G) = f4{o[j][4 * c], o[j][4 * c + 1], o[j][4 * c + 2], o[j][4 * c + 3]};
+    if (G == 0) { pp[128] = m; pp[129] = l; }
+    return;
   }
+  const float inv = l > 0.f ? 1.0f / l : 0.f;
+  uint16_t* dst = out + ((q0 + col) * 16 + h) * 128 + 4 * G;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const u2v v2 = {bfpk(o[j][4 * c] * inv, o[j][4 * c + 1] * inv), bfpk(o[j][4 * c + 2] * inv, o[j][4 * c + 3] * inv)};
+      *reinterpret_cast<u2v*>(dst + 32 * j + 8 * c) = v2;
+    }
 }
 
 // ---------------------------------------------------------------- key-split merge
