@@ -780,6 +780,64 @@ __global__ void __launch_bounds__(256) fake_quant_k_kernel(const float* __restri
   }
 }
 
+// The same for C a multiple of 4 and 16-byte aligned tensors: a workgroup takes 64 channels of one group and keeps its
+// 256 x 64 values in registers through both passes (a lane: 4 channels of the tokens 16 i + 4 w + g), so x is read once,
+// in 16-byte pieces; codes by kcode instead of an IEEE division. 32,768 tokens x 512 channels: 38 -> 20 us (of
+// 134 MB); tensors that are not aligned so, or other C, take the kernel above.
+__global__ void __launch_bounds__(256) fake_quant_k4_kernel(const float* __restrict__ x, int64_t C, float* __restrict__ out) {
+  __shared__ f4 red[2][4][16];
+  __shared__ f4 col[2][16];   // lo and scale of the 64 channels
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15;
+  const int64_t c = (int64_t)blockIdx.x * 64 + 4 * c16;
+  const int64_t at = ((int64_t)blockIdx.y * BLK + 4 * w + g) * C + c;
+  const bool in = c < C;
+  f4 v[16];
+  if (in) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = *reinterpret_cast<const f4*>(x + at + 16 * i * C);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = f4{0.f, 0.f, 0.f, 0.f};
+  }
+  f4 mn, mx;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    float lo = INFINITY, hi = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) { lo = fminf(lo, v[i][e]); hi = fmaxf(hi, v[i][e]); }
+    auto swap16 = [](float t) { return __builtin_amdgcn_permlane16_swap(__float_as_uint(t), __float_as_uint(t), false, false); };
+    auto swap32 = [](float t) { return __builtin_amdgcn_permlane32_swap(__float_as_uint(t), __float_as_uint(t), false, false); };
+    auto a = swap16(lo); lo = fminf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    a = swap32(lo); mn[e] = fminf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    auto b = swap16(hi); hi = fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+    b = swap32(hi); mx[e] = fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+  }
+  if (g == 0) { red[0][w][c16] = mn; red[1][w][c16] = mx; }
+  __syncthreads();
+  if (threadIdx.x < 64) {
+    const int t = threadIdx.x;
+    float lo = INFINITY, hi = -INFINITY;
+#pragma unroll
+    for (int ww = 0; ww < 4; ++ww) {
+      lo = fminf(lo, reinterpret_cast<const float*>(red[0][ww])[t]);
+      hi = fmaxf(hi, reinterpret_cast<const float*>(red[1][ww])[t]);
+    }
+    reinterpret_cast<float*>(col[0])[t] = f8d(f8e(lo));
+    reinterpret_cast<float*>(col[1])[t] = f8d(f8e(clamp_min_1e8(__fdiv_rn(__fsub_rn(hi, lo), 3.0f))));
+  }
+  __syncthreads();
+  if (!in) return;
+  const f4 lo = col[0][c16], sc = col[1][c16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    f4 o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)   // code sc is exact, so the fma rounds where the sum does
+      o[e] = __builtin_fmaf((float)kcode(__fsub_rn(v[i][e], lo[e]), clamp_min_1e8(sc[e])), sc[e], lo[e]);
+    *reinterpret_cast<f4*>(out + at + 16 * i * C) = o;
+  }
+}
+
 // fake_quant_v: v (N, 4, 128) fp32 -> per token y = v H (the quantizer's sequential fma chain), one bit per dim with
 // fp8 lo / scale per pair of heads, then (bit * sc8 + lo8) H with the dequantizer's chain: the V value of a
 // quantize -> dequantize round trip. A wave takes four tokens at a time through both chains on fp32 MFMA; lane (g, m)
@@ -1182,8 +1240,12 @@ int kv800_hip_fake_quant_k(const float* x, int64_t G, int64_t C, float* out, voi
   if (G == 0 || C == 0) return KV800_OK;
   KV800_REQUIRE(x && out, "fake_quant_k: null pointer");
   KV800_REQUIRE(G <= 65535 && (C + 255) / 256 <= 0x7FFFFFFF, "fake_quant_k: at most 65535 groups per call");
-  hipLaunchKernelGGL(fake_quant_k_kernel, dim3((unsigned)((C + 255) / 256), (unsigned)G), dim3(256), 0,
-                     (hipStream_t)stream, x, C, out);
+  if (C % 4 == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)out % 16) == 0)
+    hipLaunchKernelGGL(fake_quant_k4_kernel, dim3((unsigned)((C + 63) / 64), (unsigned)G), dim3(256), 0,
+                       (hipStream_t)stream, x, C, out);
+  else
+    hipLaunchKernelGGL(fake_quant_k_kernel, dim3((unsigned)((C + 255) / 256), (unsigned)G), dim3(256), 0,
+                       (hipStream_t)stream, x, C, out);
   return check_launch("fake_quant_k");
 }
 

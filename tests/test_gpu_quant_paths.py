@@ -108,3 +108,14 @@ def test_fake_quant_v_counts(hip, oracle, tokens):
     v = draw("normal", np.random.default_rng(tokens), (tokens, 4, 128)) * np.float32(1.7)
     print("fake_quant_v", tokens, flush=True)
     assert np.array_equal(hip.fake_quant_v(torch.from_numpy(v).to(DEV)).cpu().numpy(), oracle.fake_quant_v(v))
+
+
+@pytest.mark.parametrize("channels,shift", [(4, 0), (60, 0), (64, 0), (68, 0), (64, 1), (63, 0)])
+def test_fake_quant_k_channels(hip, oracle, channels, shift):
+    """Channel counts around the 64 of a workgroup, and tensors that are not 16-byte aligned (the per-channel kernel)."""
+    x = draw("channels", np.random.default_rng(channels), (3, 256, 1, channels))[:, :, 0] * np.float32(1.3)
+    raw = torch.zeros(x.size + 4, device=DEV)
+    at = raw[shift:shift + x.size].view(x.shape)
+    at.copy_(torch.from_numpy(x))
+    print("fake_quant_k", channels, shift, flush=True)
+    assert np.array_equal(hip.fake_quant_k(at).cpu().numpy(), oracle.fake_quant_k(x))
