@@ -26,13 +26,18 @@
 // each 16-key step, the key order in which the transposed reads deliver V^T. The tiles are double-buffered in LDS and
 // loaded straight into it (buffer loads with the lds modifier, through a buffer resource whose reads past the row's keys
 // return zeros; the next tile's loads are in flight while the current one is multiplied, one barrier per tile), and a
-// tile whose keys are all in range and precede the workgroup's first query is not masked.
+// tile whose keys are all in range, precede the workgroup's first query and lie in its last query's window (or are sinks)
+// is not masked.
 // Bound: matrix and VALU issue, which overlap only in part, at the clock the part holds under them (1.9 GHz here). 32 x 32
 // MFMA instead of twice as many 16 x 16 ones, with half the cross-lane steps, and the phase priorities: 8 rows x 2048
 // queries over 16K keys, whole call, 2,424 -> 2,370 -> 2,240 us (this kernel about 1.03 PFLOP/s; a library product of
 // 8192^3 reaches 1.14 on the same card).
 // Key tiles outside [first key a query of the workgroup can see, last key not in its future] are skipped: for window
-// layers only the sink keys and the keys of the window are read.
+// layers only the sink keys and the keys of the window are read, as one list (template flag WIN: its addresses cost the
+// windowless kernel 4 %). A window workgroup has 5 tiles, so its start counts as much: the row and the three key bounds
+// are found by 64-way searches side by side, behind the query loads. 8 rows x 2048 queries, window 256 + 4 sinks, whole call: 131 us
+// with a sink tile, masks on every tile and one search after the other, 115 us now (34 GFLOP, 134 MB of Q and output:
+// latency of the tiles' loads, two workgroups per CU).
 // The grid is one workgroup per (KV head, 32-query tile), numbered so that each XCD runs whole (KV head, row) runs of
 // tiles: the 64 workgroups of a 2048-query chunk walk the same key tiles together through one L2.
 #include "kv800_common.h"
@@ -88,8 +93,8 @@ __device__ __forceinline__ uint32_t bfpk(float a, float b) {
 // and the workgroups of one (KV head, row) run on one XCD, in order, so the row's key tiles are read once into that
 // XCD's L2 for its 64 query tiles. Keys come in tiles of 64, loaded into LDS as K and V rows by LDS-direct loads (no
 // register staging) and double-buffered: the next tile's loads are in flight while the current one is multiplied, one
-// barrier per tile. A tile whose keys all precede the workgroup's first query (and are all in range) needs no mask: in a
-// chunk over a long history, nearly every tile.
+// barrier per tile. A tile that every query of the workgroup sees whole needs no mask: in a chunk over a long history, nearly
+// every tile.
 constexpr int PQ = 32;      // queries per workgroup = per interface tile (tile_off counts these)
 constexpr int PPART = 132;  // floats per key-split partial of (query, head): 128 dims of o, m, l, 2 of padding
 constexpr int PMAXSPLIT = 256;
@@ -109,26 +114,35 @@ constexpr float PLAZY = 8.f;   // log2 units a query's running max may lag its s
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 constexpr int RSRC_WORD3 = 0x00020000;   // raw (untyped, unswizzled) buffer access on gfx9-family parts
 
-// first index in [0, n) with a[index] > x (a ascending; a = null: a[i] = i), n if none: a 64-way search by the whole
-// wave (lane l probes lo + l step; the count of probes <= x, from a ballot, narrows [lo, hi) 64-fold), so n = 16K
-// entries take three dependent loads instead of fourteen. All 64 lanes must be active; the result is the same in every lane.
-__device__ __forceinline__ int64_t upper(const int32_t* a, int64_t n, int64_t x) {
-  if (!a) return x < 0 ? 0 : (x + 1 < n ? x + 1 : n);   // positions = indices 0 .. n - 1
+// r[k] = first index in [0, n) with a[index] > x[k] (a ascending), n if none: NX 64-way searches by the whole wave, side
+// by side (lane l probes lo + l step; the count of probes <= x, from a ballot, narrows [lo, hi) 64-fold), so n = 4K
+// entries take two dependent loads for all of them. All 64 lanes must be active; the results are the same in every lane.
+template <int NX, typename A>
+__device__ __forceinline__ void upper(const A* a, int n, const int64_t (&x)[NX], int (&r)[NX]) {
+  int lo[NX], hi[NX];
+#pragma unroll
+  for (int k = 0; k < NX; ++k) { lo[k] = 0; hi[k] = n; }   // the answer lies in [lo, hi]
   const int lane = threadIdx.x & 63;
-  int64_t lo = 0, hi = n;   // the answer lies in [lo, hi]
-  while (hi > lo) {
-    const int64_t step = (hi - lo + 63) / 64;
-    const int64_t idx = lo + lane * step;
-    const bool le = idx < hi && (int64_t)a[idx < hi ? idx : lo] <= x;
-    const int c = __popcll(__ballot(le));   // probes 0 .. c - 1 are <= x (a ascending)
-    if (c == 0) return lo;
-    const int64_t last = lo + (int64_t)(c - 1) * step;   // a[last] <= x
-    const int64_t next = lo + (int64_t)c * step;          // the first probe > x, or past hi
-    lo = last + 1;
-    hi = next < hi ? next : hi;
-    if (step == 1) return lo;
+  for (bool more = n > 0; more;) {
+    more = false;
+    int64_t v[NX];
+#pragma unroll
+    for (int k = 0; k < NX; ++k) {
+      const int idx = lo[k] + lane * ((hi[k] - lo[k] + 63) / 64);
+      v[k] = a[idx < hi[k] ? idx : 0];
+    }
+#pragma unroll
+    for (int k = 0; k < NX; ++k) {
+      const int step = (hi[k] - lo[k] + 63) / 64;
+      const int c = __popcll(__ballot(lo[k] + lane * step < hi[k] && v[k] <= x[k]));   // probes 0 .. c - 1 are <= x
+      const int next = c == 0 ? lo[k] : lo[k] + c * step;                // the first probe > x, or past hi
+      if (c > 0) lo[k] += (c - 1) * step + 1;                            // behind the last probe <= x
+      hi[k] = step <= 1 ? lo[k] : (next < hi[k] ? next : hi[k]);
+      more = more || hi[k] > lo[k];
+    }
   }
-  return lo;
+#pragma unroll
+  for (int k = 0; k < NX; ++k) r[k] = lo[k];
 }
 
 // x's values of lanes l and l ^ 32 without an LDS round trip: v_permlane32_swap on two copies of x leaves both halves in
@@ -142,6 +156,7 @@ __device__ __forceinline__ float sum2halves(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+template <bool WIN>   // window > 0
 __global__ void __launch_bounds__(256, 2)
 prefill_kernel(const uint16_t* __restrict__ q, const int64_t* __restrict__ qsl, const int64_t* __restrict__ qpos0,
                const uint16_t* __restrict__ K, const uint16_t* __restrict__ V, const int32_t* __restrict__ kp,
@@ -158,31 +173,18 @@ prefill_kernel(const uint16_t* __restrict__ q, const int64_t* __restrict__ qsl, 
   const int g = L / (ntl * splits), h = 4 * g + w;
   const int lr = L - g * ntl * splits, sp = lr % splits;
   const int col = lane & 31, G = lane >> 5;   // query column; key / dim half
-  // ---- row of this tile: last i with tile_off[i] <= t
+  // ---- row of this tile: last i with tile_off[i] <= t (tile_off[0] = 0)
   const int64_t t = lr / splits;
-  int64_t lo = 0, hi = R;
-  while (hi - lo > 1) {
-    const int64_t mid = (lo + hi) >> 1;
-    if (tile_off[mid] <= t) lo = mid; else hi = mid;
-  }
-  const int64_t row = lo, lt = t - tile_off[row];
+  const int64_t tx[1] = {t};
+  int rows_to[1];
+  upper(tile_off, (int)R, tx, rows_to);
+  const int64_t row = max(rows_to[0], 1) - 1, lt = t - tile_off[row];
   const int64_t q0 = qsl[row] + lt * PQ;
   const int nq = (int)min((int64_t)PQ, qsl[row + 1] - q0);
   const int64_t p0 = qpos0[row] + (q0 - qsl[row]);
-  const int64_t ks = ksl[row], S = ksl[row + 1] - ks;
+  const int64_t ks = ksl[row];
+  const int S = (int)(ksl[row + 1] - ks);   // keys of 1 KB: a device holds fewer than 2^31
   const int32_t* kpr = kp ? kp + ks : nullptr;   // null: key j of the row at position j
-
-  // ---- key ranges: [0, sink_end) and [kbeg, kend)
-  const int64_t kend = upper(kpr, S, p0 + nq - 1);
-  int64_t kbeg = 0, sink_end = 0;
-  if (window > 0) {
-    kbeg = upper(kpr, S, p0 - window);
-    sink_end = min(upper(kpr, S, nsink - 1), kbeg);
-    if (kbeg <= sink_end) { kbeg = 0; sink_end = 0; }
-  }
-  const int n0 = (int)((sink_end + PK - 1) / PK), nt = n0 + (int)((kend - kbeg + PK - 1) / PK);
-  // key split sp of `splits` takes tiles [i0, i1) of the nt (all of them without a split)
-  const int per_sp = (nt + splits - 1) / splits, i0 = min(nt, sp * per_sp), i1 = min(nt, i0 + per_sp);
   // ---- the wave's queries as the B operands of S^T = K . Q^T (8 k-steps of 16 dims)
   const bool qok = col < nq;
   const int qpos = (int)(p0 + col);
@@ -190,25 +192,50 @@ prefill_kernel(const uint16_t* __restrict__ q, const int64_t* __restrict__ qsl, 
 #pragma unroll
   for (int s = 0; s < 8; ++s)
     qb[s] = qok ? *reinterpret_cast<const u4v*>(q + ((q0 + col) * 16 + h) * 128 + 16 * s + 8 * G) : u4v{0, 0, 0, 0};
+  // ---- key ranges: [0, sink_end) and [kbeg, kend)
+  const int64_t pl = p0 + nq - 1;   // the tile's last query position
+  int kend, kbeg = 0, sink_end = 0;
+  if (kpr) {
+    constexpr int NX = WIN ? 3 : 1;
+    const int64_t xs[3] = {pl, p0 - window, nsink - 1};
+    int64_t x[NX];
+    int r[NX];
+#pragma unroll
+    for (int k = 0; k < NX; ++k) x[k] = xs[k];
+    upper(kpr, S, x, r);
+    kend = r[0];
+    if (WIN) { kbeg = r[NX / 2]; sink_end = r[NX - 1]; }
+  } else {                          // positions = indices 0 .. S - 1
+    const auto first = [&](int64_t x) { return x < 0 ? 0 : (x + 1 < S ? (int)x + 1 : S); };
+    kend = first(pl);
+    if (WIN) { kbeg = first(p0 - window); sink_end = first(nsink - 1); }
+  }
+  sink_end = min(sink_end, kbeg);
+  if (kbeg <= sink_end) { kbeg = 0; sink_end = 0; }
+  // The keys as one list: entries [0, ns) the sinks, from ns on [kbeg, kend). A tile that holds both reaches from the row's
+  // first key by 32-bit byte offsets; where these do not suffice, the sinks end with a tile of their own (entries
+  // [sink_end, ns) empty). A window of 256 with 4 sinks takes 5 tiles of 64 per 32 queries instead of 6.
+  const int ns = kbeg < (1 << 20) ? sink_end : (sink_end + PK - 1) / PK * PK;
+  const int nt = (ns + (kend - kbeg) + PK - 1) / PK;
+  // key split sp of `splits` takes tiles [i0, i1) of the nt (all of them without a split)
+  const int per_sp = (nt + splits - 1) / splits, i0 = min(nt, sp * per_sp), i1 = min(nt, i0 + per_sp);
   f16v o[4];   // dims 32 j + 8 (v / 4) + 4 G + v % 4 of query col
 #pragma unroll
   for (int j = 0; j < 4; ++j)
 #pragma unroll
     for (int v = 0; v < 16; ++v) o[j][v] = 0.f;
-  float m = -1e30f, lsum = 0.f;
+  float m = qok ? -1e30f : 1e30f, lsum = 0.f;   // columns without a query never ask for a rescale
 
-  // ---- tile i's keys [k0, k0 + 64) clipped to r1: from the sink range, then from the main range
-  auto range_of = [&](int i, int64_t& k0, int64_t& r1) {
-    if (i < n0) { k0 = (int64_t)i * PK; r1 = sink_end; }
-    else { k0 = kbeg + (int64_t)(i - n0) * PK; r1 = kend; }
-  };
   int32_t skp = 0;             // the next tile's key positions (lanes < 64), stored with the tile's last reads done
   auto fetch = [&](int i, PTile& T) {
-    int64_t k0, r1;
-    range_of(i, k0, r1);
+    // tile i: list entries [c0, c0 + 64), entry c0 + j the key k0 + j, from j = cut on k0 + j + gap
+    const int c0 = i * PK;
+    const bool mixed = WIN && c0 < ns && c0 + PK > ns;
+    const int k0 = !WIN ? c0 : c0 < ns ? (mixed ? 0 : c0) : kbeg + c0 - ns;
+    const int cut = mixed ? ns - c0 : PK, gap = mixed ? kbeg - ns : 0, at = mixed ? c0 : 0;
     // the tile's K and V rows as buffers (base and size in SGPRs): a read past the row's S keys returns zeros, so every
     // staging load is issued unconditionally (keys past a range's end carry the position 0x7FFFFFFF and are masked)
-    const int nbytes = (int)(min(S - k0, (int64_t)PK) * 1024);
+    const int nbytes = min(S - k0, mixed ? kbeg + PK : PK) * 1024;
     const rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(K + (ks + k0) * 512), (short)0, nbytes,
                                                         RSRC_WORD3);
     const rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(V + (ks + k0) * 512), (short)0, nbytes,
@@ -218,13 +245,17 @@ prefill_kernel(const uint16_t* __restrict__ q, const int64_t* __restrict__ qsl, 
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int j = 16 * r + 4 * w + (lane >> 4), qs = lane & 15;
-      const int base = j * 1024 + g * 256;
+      const int base = (at + j + (j >= cut ? gap : 0)) * 1024 + g * 256;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (__attribute__((address_space(3))) void*)&T.k[(16 * r + 4 * w) * 128],
                                                16, base + 16 * kswz(j, qs), 0, 0, 0);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (__attribute__((address_space(3))) void*)&T.v[(16 * r + 4 * w) * 128],
                                                16, base + 16 * vswz(j, qs), 0, 0, 0);
     }
-    if (tid < PK) skp = (k0 + tid < r1) ? (kpr ? kpr[k0 + tid] : (int32_t)(k0 + tid)) : 0x7FFFFFFF;
+    if (tid < PK) {
+      const int key = k0 + at + tid + (tid >= cut ? gap : 0);
+      const bool in = key < (WIN && c0 + tid < ns ? sink_end : kend);
+      skp = in ? (kpr ? kpr[key] : key) : 0x7FFFFFFF;
+    }
     // the loads write T behind the compiler's view of the buffer: its address escapes here
     asm volatile("" ::"s"((uint32_t)(uintptr_t)&T) : "memory");
   };
@@ -250,20 +281,19 @@ prefill_kernel(const uint16_t* __restrict__ q, const int64_t* __restrict__ qsl, 
         sc[nb] = mfma_bf(a, qb[s], s == 0 ? zero : sc[nb]);
       }
     }
-    // ---- mask, scale, online softmax (the lane's 32 keys). No mask when every key of the tile is in range and precedes
-    // the workgroup's first query (quantized layers: no window).
-    int64_t tk0, tr1;
-    range_of(i, tk0, tr1);
-    const bool full = window <= 0 && tk0 + PK <= tr1 && (int64_t)T.kp[PK - 1] <= p0;
+    // ---- mask, scale, online softmax (the lane's 32 keys). No mask when every key of the tile is in range, precedes the
+    // workgroup's first query and is a sink or inside the window of its last one.
+    const int64_t kfirst = T.kp[0], klast = T.kp[PK - 1];   // ascending; klast is 0x7FFFFFFF if entries are missing
+    const bool full = klast <= p0 && (!WIN || kfirst > pl - window || klast < nsink);
     if (!full) {
-      const int wlo = window > 0 ? (int)max((int64_t)qpos - window, (int64_t)INT32_MIN) : INT32_MIN;
-      const int ns = window > 0 ? (int)nsink : 0;
+      const int wlo = WIN ? (int)max((int64_t)qpos - window, (int64_t)INT32_MIN) : INT32_MIN;
+      const int nsk = WIN ? (int)nsink : 0;
 #pragma unroll
       for (int nb = 0; nb < 2; ++nb) {
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
           const int kpos = T.kp[nb * 32 + 8 * (v >> 2) + 4 * G + (v & 3)];
-          const bool keep = qok & (kpos <= qpos) & ((kpos > wlo) | (kpos < ns));
+          const bool keep = qok & (kpos <= qpos) & ((kpos > wlo) | (kpos < nsk));
           sc[nb][v] = keep ? sc[nb][v] : -INFINITY;
         }
       }
@@ -433,7 +463,7 @@ int kv800_hip_prefill_split(const uint16_t* q, const int64_t* qsl, const int64_t
                   (long long)part_floats, (long long)(T * 16 * splits * PPART));
   }
   const float scale_log2 = 0.088388347648318440f * 1.4426950408889634f;   // 128^-0.5 * log2(e)
-  hipLaunchKernelGGL(prefill_kernel, dim3((unsigned)(ntiles * 4 * splits)), dim3(256), 0, (hipStream_t)stream, q, qsl,
+  hipLaunchKernelGGL(window > 0 ? prefill_kernel<true> : prefill_kernel<false>, dim3((unsigned)(ntiles * 4 * splits)), dim3(256), 0, (hipStream_t)stream, q, qsl,
                      qpos0, K, V, kp, ksl, tile_off, R, window, nsink, scale_log2, out, (int)splits,
                      splits > 1 ? part : (float*)nullptr);
   int rc = check_launch("prefill");
