@@ -132,8 +132,9 @@ C2_B, C2_N, C2_EBS = 64, 2048, 128
 C2_NQ = (C2_N - 128) // 256                         # 7 flushed sub-blocks per sequence (kv800.py:433 flush rule)
 C2_READ = C2_B * C2_NQ * 256 * 4 * 128 * 2 * 2      # bf16 K + V gathered from the exact pages
 C2_WRITE = C2_B * C2_NQ * 51200
-C2_FMA = C2_B * C2_NQ * 256 * 4 * 16 * 688          # fp32 fma of the bit-exact V Hadamard chains: 688 per lane's 8
-                                                    # outputs (16 lanes per head row), 86 per output
+C2_FMA = C2_B * C2_NQ * 256 * 4 * 16 * 688          # fp32 fma of the V Hadamard as sequential chains with shared
+                                                    # prefixes, 86 per output: a measure of the work, of which the
+                                                    # kernel forms most on the matrix cores (fma_frac may exceed 1)
 FMA_PEAK = 256 * 64 * 2.4e9                         # non-packed fp32 fma/s: 256 CUs x 64 lanes x 2.4 GHz
 
 

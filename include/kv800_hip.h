@@ -70,7 +70,7 @@ int kv800_hip_flush(const uint16_t* epool, const int64_t* eoff, int64_t eoff_str
                     void* stream);
 
 /* kv800_hip_flush with the same arguments and bytes, organised for the latency of a flush of few sub-blocks (a decode
- * step flushes at most one per row, usually one or two per layer): one token per V wave, each K row read once. Use
+ * step flushes at most one per row, usually one or two per layer): four tokens per V wave, each K row read once. Use
  * kv800_hip_flush when many sub-blocks are flushed at once (prefill chunks). */
 int kv800_hip_flush_latency(const uint16_t* epool, const int64_t* eoff, int64_t eoff_stride, int64_t ebs, int64_t e_hs,
                             int64_t e_ts, int64_t e_v, uint8_t* qpool, const int64_t* qbt, int64_t qbt_stride,
