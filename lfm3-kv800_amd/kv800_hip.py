@@ -394,11 +394,21 @@ class PrefillRows:
         R = self.R = len(qpos0)
         if len(qsl) != R + 1 or len(ksl) != R + 1:
             raise ValueError("qsl and ksl need R + 1 entries")
+        if any(x[0] or any(b < a for a, b in zip(x, x[1:])) for x in (qsl, ksl)):
+            raise ValueError("qsl and ksl must start at 0 and not decrease")
         tiles = [0]
         for a, b in zip(qsl, qsl[1:]):
             tiles.append(tiles[-1] + (b - a + 31) // 32)   # 32-query tiles, one workgroup per tile and KV head
         self.qsl, self.ksl, self.qpos0, self.ntiles, self.dev = qsl, ksl, qpos0, tiles[-1], dev
         self._host, self._meta = qsl + ksl + qpos0 + tiles, None
+
+    def need_counts(self, counts):
+        """Each row's keys must be counts[r] rows before its new ones: what the assembly launches read and write."""
+        if any(x < 0 for x in self.qpos0):
+            raise ValueError("history lengths must be >= 0")
+        q, s = self.qsl, self.ksl
+        if any(s[r + 1] - s[r] != c + q[r + 1] - q[r] for r, c in enumerate(counts)):
+            raise ValueError("ksl does not match the rows' history and new rows")
 
     def ptrs(self):
         """Device pointers of (qsl, ksl, qpos0, tiles); the tensor behind them lives as long as this object."""
@@ -500,8 +510,7 @@ def prefill_keys(P, rows, k, v, cos_t, sin_t):
     L = ops()
     dev = P.epool.device
     R, prev = rows.R, rows.qpos0
-    if any(x < 0 for x in prev):
-        raise ValueError("history lengths must be >= 0")
+    rows.need_counts(prev)
     k, v = _new_rows(k, v, rows.qsl[-1], dev)
     cos_t, sin_t = _rope32(cos_t, sin_t, dev)
     K = torch.empty(rows.ksl[-1], 4, 128, dtype=torch.bfloat16, device=dev)
@@ -522,12 +531,18 @@ def prefill_keys(P, rows, k, v, cos_t, sin_t):
     return K, V
 
 
+def window_counts(prev, win, nsink):
+    """Keys that a window layer holds of histories of prev[r] positions: the last win - 1, and the sinks before them."""
+    return [min(n, win - 1) + min(nsink, max(0, n - (win - 1))) for n in prev]
+
+
 def window_keys(P, rows, k, v, cos_t, sin_t, win, nsink):
     """The same for a window layer (kv800_hip_window_keys): sinks, kept exact rows, new rows; returns (K, V, positions
     (S,) int32). cos_t None: keys as stored."""
     L = ops()
     dev = P.epool.device
     R = rows.R
+    rows.need_counts(window_counts(rows.qpos0, win, nsink))
     k, v = _new_rows(k, v, rows.qsl[-1], dev)
     if cos_t is not None:
         cos_t, sin_t = _rope32(cos_t, sin_t, dev)
@@ -536,7 +551,8 @@ def window_keys(P, rows, k, v, cos_t, sin_t, win, nsink):
     kp = torch.empty(rows.ksl[-1], dtype=torch.int32, device=dev)
     if not R or not rows.ksl[-1]:
         return K, V, kp
-    eoff = P.eoff if P.eoff.stride(-1) == 1 else P.eoff.contiguous()
+    eoff = P.eoff.to(torch.int64)   # any integer type and stride, as for an index
+    eoff = eoff if eoff.stride(-1) == 1 else eoff.contiguous()
     _need(P.epool, "epool", torch.bfloat16, dev); _need(eoff, "eoff", torch.int64, dev)
     if eoff.shape[0] < R or any(n > 0 and (n - 1) // int(P.ebs) >= eoff.shape[1] for n in rows.qpos0):
         raise IndexError("eoff does not cover the rows' positions")
@@ -547,8 +563,8 @@ def window_keys(P, rows, k, v, cos_t, sin_t, win, nsink):
     sink_elems = 0
     if nsink:
         _need(P.sk, "sk", torch.bfloat16, dev); _need(P.sv, "sv", torch.bfloat16, dev)
-        _need(P.skoff, "skoff", torch.int64, dev); _need(P.svoff, "svoff", torch.int64, dev)
-        skoff, svoff = P.skoff.contiguous(), P.svoff.contiguous()
+        skoff, svoff = P.skoff.to(torch.int64).contiguous(), P.svoff.to(torch.int64).contiguous()
+        _need(skoff, "skoff", torch.int64, dev); _need(svoff, "svoff", torch.int64, dev)
         if skoff.shape[0] < R or svoff.shape[0] < R:
             raise IndexError("skoff / svoff must cover the rows")
         s.sk, s.sv, s.skoff, s.svoff = P.sk.data_ptr(), P.sv.data_ptr(), skoff.data_ptr(), svoff.data_ptr()

@@ -386,6 +386,8 @@ def _ranges(starts, counts):
 
 def _rows(qsl, counts, prev, dev):
     """PrefillRows of rows with `counts` keys before their new rows qsl[i] .. qsl[i + 1], from position prev[i] on."""
+    if any(n < 0 for n in prev):
+        raise ValueError("history lengths must be >= 0")
     ksl = [0]
     for i, c in enumerate(counts):
         ksl.append(ksl[-1] + c + qsl[i + 1] - qsl[i])
@@ -428,7 +430,6 @@ def prefill_window_rows(P, q, k, v, qsl, prev, cos_t, sin_t):
     mask (and the sinks). qsl / prev are host sequences. Returns (T, 16, 128) bf16."""
     prev, qsl = [int(x) for x in prev], [int(x) for x in qsl]
     nsink = kv800.NSINK if P.sk is not None else 0
-    kept = [min(n, kv800.WIN - 1) + min(nsink, max(0, n - (kv800.WIN - 1))) for n in prev]
-    rows = _rows(qsl, kept, prev, q.device)
+    rows = _rows(qsl, kv800_hip.window_counts(prev, kv800.WIN, nsink), prev, q.device)
     K, V, kp = kv800_hip.window_keys(P, rows, k, v, cos_t, sin_t, kv800.WIN, nsink)
     return kv800_hip.prefill_rows(q, rows, K, V, kp, window=kv800.WIN, nsink=nsink)

@@ -1,0 +1,36 @@
+"""Row geometry of prefill calls on the host: what the key assembly's launches would read or write out of range is
+refused before any launch, as the gathers refused it."""
+import pytest
+import torch
+
+CPU = torch.device("cpu")
+
+
+@pytest.mark.parametrize("qsl,ksl", [([0, 5, 3], [0, 5, 8]), ([0, 3, 5], [0, 8, 5]), ([1, 3, 5], [0, 3, 5]),
+                                     ([0, 3, 5], [2, 5, 7]), ([0, 3], [0, 3, 5])])
+def test_starts_that_are_no_prefix_sums(qsl, ksl):
+    from lfm3_kv800_amd import kv800_hip
+    with pytest.raises(ValueError):
+        kv800_hip.PrefillRows(qsl, ksl, [0, 0], CPU)
+
+
+@pytest.mark.parametrize("call", ["prefill_quant_rows", "prefill_window_rows"])
+@pytest.mark.parametrize("qsl,prev", [([0, 5, 3], [2, 0]), ([0, 3, 5], [4, -1])])
+def test_calls_refuse_bad_rows(call, qsl, prev):
+    from lfm3_kv800_amd import vllm_cache
+    import lfm3_kv800_amd.kv800 as kv
+    x = torch.zeros(5, 4, 128, dtype=torch.bfloat16)
+    t = torch.zeros(8, 32, dtype=torch.bfloat16)
+    with pytest.raises(ValueError):
+        getattr(vllm_cache, call)(kv.Paged(), x.repeat(1, 4, 1), x, x, qsl, prev, t, t)
+
+
+def test_counts_match_the_rows():
+    from lfm3_kv800_amd import kv800_hip
+    prev = [0, 255, 256, 300]
+    assert kv800_hip.window_counts(prev, 256, 4) == [0, 255, 256, 259]
+    assert kv800_hip.window_counts(prev, 256, 0) == [0, 255, 255, 255]
+    rows = kv800_hip.PrefillRows([0, 2, 2, 5, 6], [0, 2, 257, 516, 776], prev, CPU)
+    rows.need_counts(kv800_hip.window_counts(prev, 256, 4))
+    with pytest.raises(ValueError):
+        rows.need_counts(kv800_hip.window_counts(prev, 256, 0))
