@@ -379,9 +379,15 @@ prefill_kernel(const uint16_t* __restrict__ q, const int64_t* __restrict__ qsl, 
 }
 
 // ---------------------------------------------------------------- key-split merge
-// One wave per (query, head). Lanes read the splits' (m, l) in parallel: M = max m_s and L = sum l_s 2^(m_s - M) by
-// wave reductions; then lane holds dims 2 lane, 2 lane + 1 and sums o_s 2^(m_s - M) over the splits, eight loads in
-// flight; out = bf16(O / L) (a split without keys has l = 0 and o = 0).
+// W waves per (query, head). Lanes read the splits' (m, l) in parallel: M = max m_s and L = sum l_s 2^(m_s - M) by
+// wave reductions; then lane holds dims 2 lane, 2 lane + 1 and sums o_s 2^(m_s - M) over its wave's splits, the first
+// loads in flight during the reductions, the waves' sums added through LDS; out = bf16(O / L) (a split without keys has
+// l = 0 and o = 0). Bound: latency, of the partials other XCDs wrote. 4 waves per pair where one would leave most CUs
+// without a workgroup (up to 64 queries) and each of the 4 has several partials: whole attention call, 16 queries x 16K
+// keys in 64 splits 22.0 -> 16.9 us, 32 queries 24.9 -> 20.4, 64 queries x 4K keys in 32 splits 21.8 -> 21.1; but 128 queries
+// x 4K in 8 splits 22.4 -> 26.3, 64 queries x 16K in 16 splits 30.9 -> 31.9, so these keep one wave.
+constexpr int64_t MERGE_WIDE_PAIRS = 1024;
+constexpr int MERGE_WIDE_SPLITS = 17;
 __device__ __forceinline__ float wave_max(float x) {
 #pragma unroll
   for (int k = 1; k < 64; k <<= 1) x = fmaxf(x, __shfl_xor(x, k, 64));
@@ -392,33 +398,58 @@ __device__ __forceinline__ float wave_sum(float x) {
   for (int k = 1; k < 64; k <<= 1) x += __shfl_xor(x, k, 64);
   return x;
 }
+template <int W>   // waves per pair
 __global__ void __launch_bounds__(256)
 prefill_merge_kernel(const float* __restrict__ part, int64_t pairs, int splits, uint16_t* __restrict__ out) {
-  const int64_t pr = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (pr >= pairs) return;   // uniform over the wave
-  const int lane = threadIdx.x & 63;
+  constexpr int N = W == 1 ? 8 : 16;   // partials in flight per wave
+  __shared__ float2 red[4][64];
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, sub = w % W;
+  const int64_t pr = (int64_t)blockIdx.x * (4 / W) + w / W;
+  if (W == 1 && pr >= pairs) return;   // uniform over the wave; with W = 4 the grid is exact
   const float* pp = part + pr * splits * PPART;
-  float M = -INFINITY;
-  for (int s = lane; s < splits; s += 64) M = fmaxf(M, pp[s * PPART + 128]);
-  M = wave_max(M);
-  float Ls = 0.f;
-  for (int s = lane; s < splits; s += 64) Ls += __builtin_amdgcn_exp2f(pp[s * PPART + 128] - M) * pp[s * PPART + 129];
-  Ls = wave_sum(Ls);
-  float o0 = 0.f, o1 = 0.f;
-  for (int s0 = 0; s0 < splits; s0 += 8) {
-    float mv[8];
-    float2 av[8];
+  float mv[N];
+  float2 av[N];
+  const auto load = [&](int s0) {   // splits s0 + W k
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const int sk = s0 + k < splits ? s0 + k : s0;   // past the last split: a repeat, weighted 0 below
-      mv[k] = s0 + k < splits ? pp[sk * PPART + 128] : -INFINITY;
+    for (int k = 0; k < N; ++k) {
+      const int s = s0 + W * k, sk = s < splits ? s : 0;   // past the last split: a repeat, weighted 0 below
+      mv[k] = s < splits ? pp[sk * PPART + 128] : -INFINITY;
       av[k] = *reinterpret_cast<const float2*>(pp + sk * PPART + 2 * lane);
     }
+  };
+  load(sub);
+  float2 ml[PMAXSPLIT / 64];   // (m, l) of splits lane + 64 i
+  float M = -INFINITY, Ls = 0.f;
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
+  for (int i = 0; i < PMAXSPLIT / 64; ++i) {
+    const int s = lane + 64 * i;
+    ml[i] = s < splits ? *reinterpret_cast<const float2*>(pp + s * PPART + 128) : make_float2(-INFINITY, 0.f);
+    M = fmaxf(M, ml[i].x);
+  }
+  M = wave_max(M);
+#pragma unroll
+  for (int i = 0; i < PMAXSPLIT / 64; ++i) Ls += __builtin_amdgcn_exp2f(ml[i].x - M) * ml[i].y;
+  Ls = wave_sum(Ls);
+  float o0 = 0.f, o1 = 0.f;
+  for (int s0 = sub;;) {
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
       const float wgt = __builtin_amdgcn_exp2f(mv[k] - M);
       o0 += wgt * av[k].x;
       o1 += wgt * av[k].y;
+    }
+    s0 += W * N;
+    if (s0 >= splits) break;   // uniform over the wave
+    load(s0);
+  }
+  if (W > 1) {
+    red[w][lane] = make_float2(o0, o1);
+    __syncthreads();
+    if (sub) return;
+#pragma unroll
+    for (int k = 1; k < W; ++k) {
+      o0 += red[w + k][lane].x;
+      o1 += red[w + k][lane].y;
     }
   }
   const float inv = Ls > 0.f ? 1.0f / Ls : 0.f;
@@ -469,8 +500,9 @@ int kv800_hip_prefill_split(const uint16_t* q, const int64_t* qsl, const int64_t
   int rc = check_launch("prefill");
   if (rc != KV800_OK || splits == 1 || T == 0) return rc;
   const int64_t pairs = T * 16;
-  hipLaunchKernelGGL(prefill_merge_kernel, dim3((unsigned)((pairs + 3) / 4)), dim3(256), 0, (hipStream_t)stream, part,
-                     pairs, (int)splits, out);
+  const bool wide = pairs <= MERGE_WIDE_PAIRS && splits >= MERGE_WIDE_SPLITS;
+  hipLaunchKernelGGL(wide ? prefill_merge_kernel<4> : prefill_merge_kernel<1>, dim3((unsigned)(wide ? pairs : (pairs + 3) / 4)),
+                     dim3(256), 0, (hipStream_t)stream, part, pairs, (int)splits, out);
   return check_launch("prefill_merge");
 }
 
