@@ -372,16 +372,25 @@ def rope_rows(k, pos, cos_t, sin_t):
 
 
 PREFILL_SPLIT_BELOW = 256   # workgroups (query tiles x 4 KV heads) under which the key range is split
-PREFILL_SPLIT_TARGET = 512  # workgroups a split grid aims at (two per CU)
+PREFILL_SPLIT_TARGETS = (512, 256)  # workgroups a split grid aims at: two per CU over long rows, else one
+PREFILL_SPLIT_TILES = 16    # 64-key tiles per split from which two per CU pay
 
 
 def prefill_splits(tiles, max_key_tiles):
     """Key splits of one prefill launch: 1 when its tiles x 4 workgroups nearly fill the GPU, else enough for about
-    PREFILL_SPLIT_TARGET workgroups, with at least two 64-key tiles per split and at most 64 splits."""
+    512 workgroups, or 256 when that many would have fewer than PREFILL_SPLIT_TILES key tiles each (two workgroups on a CU
+    gain about 15 % per tile, against twice the partials), with at least two 64-key tiles per split and at most 64 splits.
+    512 / 256 workgroups, whole attention call in us: 64 queries x 16K keys 33 / 26, 128 x 4K 27.9 / 23.0, 128 x 16K
+    39.1 / 34.7, 256 x 4K 30.1 / 27.1, 512 x 1K 26.2 / 21.8; but 256 x 16K 51.8 / 53.1, 512 x 16K 82 / 101, 128 x 64K
+    86 / 94."""
     w = 4 * tiles
     if w >= PREFILL_SPLIT_BELOW or max_key_tiles < 4:
         return 1
-    return int(max(1, min(64, -(-PREFILL_SPLIT_TARGET // w), max_key_tiles // 2)))
+    for target in PREFILL_SPLIT_TARGETS:
+        s = int(max(1, min(64, -(-target // w), max_key_tiles // 2)))
+        if max_key_tiles >= PREFILL_SPLIT_TILES * s:
+            break
+    return s
 
 
 class PrefillRows:
