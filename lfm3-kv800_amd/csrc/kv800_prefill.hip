@@ -21,9 +21,10 @@
 //   O^T += V^T . P^T (dims x queries): A = V^T read from the V rows by ds_read_b64_tr_b16, B = the lane's own
 //                    probabilities.
 // Both results keep one query per lane column (l % 32), so the softmax statistics of a query live in two lanes and are
-// combined with one cross-lane step, and the O rescale (lazy: only when a query's running max grows by more than PLAZY)
-// needs no data movement. P^T's B operand is the lane's 8 probabilities of keys 4 G + i and 8 + 4 G + i (G = l / 32) of
-// each 16-key step, the key order in which the transposed reads deliver V^T. The tiles are double-buffered in LDS and
+// combined with one cross-lane step, and the O rescale (when a query's running max grows, over one long list of keys only
+// when it grows by more than PLAZY; 16 queries at a time) needs no data movement. P^T's B operand is the lane's 8
+// probabilities of keys 4 G + i and 8 + 4 G + i (G = l / 32) of each 16-key step, the key order in which the transposed
+// reads deliver V^T. The tiles are double-buffered in LDS and
 // loaded straight into it (buffer loads with the lds modifier, through a buffer resource whose reads past the row's keys
 // return zeros; the next tile's loads are in flight while the current one is multiplied, one barrier per tile), and a
 // tile whose keys are all in range, precede the workgroup's first query and lie in its last query's window (or are sinks)
@@ -36,7 +37,7 @@
 // layers only the sink keys and the keys of the window are read, as one list (template flag WIN: its addresses cost the
 // windowless kernel 4 %). A window workgroup has 5 tiles, so its start counts as much: the row and the three key bounds
 // are found by 64-way searches side by side, behind the query loads. 8 rows x 2048 queries, window 256 + 4 sinks, whole call: 131 us
-// with a sink tile, masks on every tile and one search after the other, 115 us now (34 GFLOP, 134 MB of Q and output:
+// with a sink tile, masks on every tile and one search after the other, 117 us now (34 GFLOP, 134 MB of Q and output:
 // latency of the tiles' loads, two workgroups per CU).
 // The grid is one workgroup per (KV head, 32-query tile), numbered so that each XCD runs whole (KV head, row) runs of
 // tiles: the 64 workgroups of a 2048-query chunk walk the same key tiles together through one L2.
@@ -110,7 +111,13 @@ struct alignas(16) PTile {
 };
 __device__ __forceinline__ int kswz(int j, int p) { return p ^ (j & 15); }
 __device__ __forceinline__ int vswz(int j, int p) { return p ^ (2 * (j & 7)); }
-constexpr float PLAZY = 8.f;   // log2 units a query's running max may lag its scores (p <= 2^8 in bf16)
+// Log2 units a query's running max may lag its scores (p <= 2^8 in bf16) where it sees the keys as one long list. A window
+// workgroup or a key split sees a few tiles, and there the max is kept exact (no lag): the largest key's probability is then
+// 1, without a bf16 rounding, while a max of the first tile that later keys just exceed puts these where the rounding is
+// coarsest. Error against 64 bits with the lag / without: window 256 + 4 sinks 2.24e-3 / 1.85e-3, split rows 2.06-2.21e-3 /
+// 1.71-1.77e-3 (1.66e-3 is the rounding of the output alone); time 113.7 / 116.4 us (8 x 2048 queries, window), 26.0 / 26.7
+// us (64 queries x 16K keys, 32 splits). Over 16K keys unsplit, 2.204e-3, no lag would rescale in most tiles.
+constexpr float PLAZY = 8.f;
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 constexpr int RSRC_WORD3 = 0x00020000;   // raw (untyped, unswizzled) buffer access on gfx9-family parts
 
@@ -226,6 +233,7 @@ prefill_kernel(const uint16_t* __restrict__ q, const int64_t* __restrict__ qsl, 
     for (int v = 0; v < 16; ++v) o[j][v] = 0.f;
   float m = qok ? -1e30f : 1e30f, lsum = 0.f;   // columns without a query never ask for a rescale
 
+  const float lazy = WIN || part ? 0.f : PLAZY;
   int32_t skp = 0;             // the next tile's key positions (lanes < 64), stored with the tile's last reads done
   auto fetch = [&](int i, PTile& T) {
     // tile i: list entries [c0, c0 + 64), entry c0 + j the key k0 + j, from j = cut on k0 + j + gap
@@ -305,8 +313,10 @@ prefill_kernel(const uint16_t* __restrict__ q, const int64_t* __restrict__ qsl, 
 #pragma unroll
       for (int v = 0; v < 16; v += 2) tmax = fmaxf(fmaxf(tmax, sc[nb][v]), sc[nb][v + 1]);
     tmax = max2halves(tmax) * scale_log2;   // scale > 0: the max of the scaled scores
-    if (__any(tmax > m + PLAZY)) {   // rescale only when a query's max outgrows its state (wave-uniform)
-      const float mnew = fmaxf(m, tmax);
+    // a query outgrows its state: its 16-query half of the columns rescales (the branch is wave-uniform)
+    const uint64_t grow = __ballot(tmax > m + lazy);
+    if (grow) {
+      const float mnew = (grow & (col < 16 ? 0x0000FFFF0000FFFFull : 0xFFFF0000FFFF0000ull)) ? fmaxf(m, tmax) : m;
       const float alpha = __builtin_amdgcn_exp2f(m - mnew);
       m = mnew;
       lsum *= alpha;
