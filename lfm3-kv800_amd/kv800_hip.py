@@ -400,6 +400,9 @@ class PrefillRows:
 
     def __init__(self, qsl, ksl, qpos0, dev):
         qsl, ksl, qpos0 = [int(x) for x in qsl], [int(x) for x in ksl], [int(x) for x in qpos0]
+        dev = torch.device(dev)
+        if dev.type == "cuda" and dev.index is None:
+            dev = torch.device("cuda", torch.cuda.current_device())
         R = self.R = len(qpos0)
         if len(qsl) != R + 1 or len(ksl) != R + 1:
             raise ValueError("qsl and ksl need R + 1 entries")
@@ -410,6 +413,11 @@ class PrefillRows:
             tiles.append(tiles[-1] + (b - a + 31) // 32)   # 32-query tiles, one workgroup per tile and KV head
         self.qsl, self.ksl, self.qpos0, self.ntiles, self.dev = qsl, ksl, qpos0, tiles[-1], dev
         self._host, self._meta = qsl + ksl + qpos0 + tiles, None
+
+    def need_device(self, dev):
+        """The launches read the geometry through raw pointers: it must be on their tensors' device."""
+        if self.dev != dev:
+            raise ValueError(f"the row geometry is on {self.dev}, the call's tensors on {dev}")
 
     def need_counts(self, counts):
         """Each row's keys must be counts[r] rows before its new ones: what the assembly launches read and write."""
@@ -441,6 +449,7 @@ def prefill_rows(q, rows, K, V, kp, window=0, nsink=0, splits=None):
     """prefill with the row geometry already in a PrefillRows."""
     L = ops()
     dev = q.device
+    rows.need_device(dev)
     q, K, V = q.contiguous(), K.contiguous(), V.contiguous()
     _need(q, "q", torch.bfloat16, dev); _need(K, "K", torch.bfloat16, dev); _need(V, "V", torch.bfloat16, dev)
     qsl, ksl, R = rows.qsl, rows.ksl, rows.R
@@ -519,6 +528,7 @@ def prefill_keys(P, rows, k, v, cos_t, sin_t):
     L = ops()
     dev = P.epool.device
     R, prev = rows.R, rows.qpos0
+    rows.need_device(dev)
     rows.need_counts(prev)
     k, v = _new_rows(k, v, rows.qsl[-1], dev)
     cos_t, sin_t = _rope32(cos_t, sin_t, dev)
@@ -551,6 +561,7 @@ def window_keys(P, rows, k, v, cos_t, sin_t, win, nsink):
     L = ops()
     dev = P.epool.device
     R = rows.R
+    rows.need_device(dev)
     rows.need_counts(window_counts(rows.qpos0, win, nsink))
     k, v = _new_rows(k, v, rows.qsl[-1], dev)
     if cos_t is not None:

@@ -34,3 +34,31 @@ def test_counts_match_the_rows():
     rows.need_counts(kv800_hip.window_counts(prev, 256, 4))
     with pytest.raises(ValueError):
         rows.need_counts(kv800_hip.window_counts(prev, 256, 0))
+
+
+class Calls:
+    """A library whose entry points only note that they were called."""
+    def __init__(self):
+        self.made = []
+
+    def __getattr__(self, name):
+        return lambda *a: self.made.append(name) or 0
+
+
+@pytest.mark.parametrize("call", ["prefill_quant_rows", "prefill_window_rows"])
+def test_calls_refuse_queries_of_another_device(monkeypatch, call):
+    """The row geometry is made on the queries' device and the assembly reads it on the cache's."""
+    from lfm3_kv800_amd import kv800_hip, vllm_cache
+    import lfm3_kv800_amd.kv800 as kv
+    lib = Calls()
+    monkeypatch.setattr(kv800_hip, "ops", lambda: lib)
+    monkeypatch.setattr(kv800_hip, "_stream", lambda dev: None)
+    bf = dict(dtype=torch.bfloat16)
+    P = kv.Paged(epool=torch.zeros(1, 4, 64, 256, **bf), eoff=torch.zeros(1, 1, dtype=torch.int64), ebs=64, e_hs=64 * 256,
+                 e_ts=256, e_v=128, NQ=torch.zeros(1, dtype=torch.int32))
+    x, t = torch.zeros(5, 4, 128, **bf), torch.zeros(16, 32, **bf)
+    with pytest.raises(ValueError):
+        getattr(vllm_cache, call)(P, torch.empty(5, 16, 128, device="meta", **bf), x, x, [0, 5], [7], t, t)
+    assert lib.made == []
+    getattr(vllm_cache, call)(P, x.repeat(1, 4, 1), x, x, [0, 5], [7], t, t)
+    assert len(lib.made) == 2   # the assembly and the attention
