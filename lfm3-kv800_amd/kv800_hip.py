@@ -135,6 +135,10 @@ def _stream(dev):
     return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
 
 
+def _stream_key(dev):
+    return torch.cuda.current_stream(dev).cuda_stream if dev.type == "cuda" else 0
+
+
 def _extent(t):
     """Elements from t's first element to the end of its storage (what the kernels may address from data_ptr)."""
     return t.untyped_storage().nbytes() // t.element_size() - t.storage_offset()
@@ -394,7 +398,7 @@ def prefill_splits(tiles, max_key_tiles):
 
 
 class PrefillRows:
-    """Row geometry of a prefill call, on the host and (one upload) on the device: row r's queries / new rows
+    """Row geometry of a prefill call, on the host and (one upload per stream) on the device: row r's queries / new rows
     [qsl[r], qsl[r + 1]) from position qpos0[r] on, its keys [ksl[r], ksl[r + 1]), and the prefix sums of its 32-query
     tiles."""
 
@@ -412,7 +416,7 @@ class PrefillRows:
         for a, b in zip(qsl, qsl[1:]):
             tiles.append(tiles[-1] + (b - a + 31) // 32)   # 32-query tiles, one workgroup per tile and KV head
         self.qsl, self.ksl, self.qpos0, self.ntiles, self.dev = qsl, ksl, qpos0, tiles[-1], dev
-        self._host, self._meta = qsl + ksl + qpos0 + tiles, None
+        self._host, self._meta = qsl + ksl + qpos0 + tiles, {}
 
     def need_device(self, dev):
         """The launches read the geometry through raw pointers: it must be on their tensors' device."""
@@ -428,10 +432,13 @@ class PrefillRows:
             raise ValueError("ksl does not match the rows' history and new rows")
 
     def ptrs(self):
-        """Device pointers of (qsl, ksl, qpos0, tiles); the tensor behind them lives as long as this object."""
-        if self._meta is None:
-            self._meta = host_to_device(self._host, torch.int64, self.dev)
-        p, n = self._meta.data_ptr(), self.R + 1
+        """Device pointers of (qsl, ksl, qpos0, tiles) for launches on the current stream; the tensor behind them lives as
+        long as this object. One upload per stream: another stream would neither wait for it nor keep its memory."""
+        key = _stream_key(self.dev)
+        meta = self._meta.get(key)
+        if meta is None:   # of two threads on one stream both take the first's
+            meta = self._meta.setdefault(key, host_to_device(self._host, torch.int64, self.dev))
+        p, n = meta.data_ptr(), self.R + 1
         return tuple(ctypes.c_void_p(p + 8 * i) for i in (0, n, 2 * n, 3 * n - 1))
 
 

@@ -62,3 +62,17 @@ def test_calls_refuse_queries_of_another_device(monkeypatch, call):
     assert lib.made == []
     getattr(vllm_cache, call)(P, x.repeat(1, 4, 1), x, x, [0, 5], [7], t, t)
     assert len(lib.made) == 2   # the assembly and the attention
+
+
+def test_one_upload_per_stream(monkeypatch):
+    from lfm3_kv800_amd import kv800_hip
+    stream = [1]
+    monkeypatch.setattr(kv800_hip, "_stream_key", lambda dev: stream[0], raising=False)
+    rows = kv800_hip.PrefillRows([0, 5], [0, 12], [7], CPU)
+    at = lambda: [p.value for p in rows.ptrs()]
+    first = at()
+    stream[0] = 2
+    second = at()
+    assert set(first).isdisjoint(second) and at() == second
+    stream[0] = 1
+    assert at() == first
