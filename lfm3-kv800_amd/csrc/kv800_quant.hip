@@ -15,6 +15,8 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
+
 #include "kv800_common.h"
 #include "../../include/kv800_hip.h"
 
@@ -1120,6 +1122,7 @@ __global__ void __launch_bounds__(256) history_kernel(kv800_paged_t P, const uin
 // 0 .. min(nsink, lo) - 1. Rows outside the pools are zeros. A workgroup copies WIN_ROWS rows, 32 units a row.
 // 8 rows of 2,048 new tokens over a full window: the whole call 555 -> 134 us.
 constexpr int WIN_ROWS = 32;
+constexpr int64_t MAX_GRID_Y = 65535;
 __global__ void __launch_bounds__(256) window_keys_kernel(kv800_paged_t P, const uint16_t* __restrict__ cos_t,
                                                           const uint16_t* __restrict__ sin_t, int64_t rope_rows,
                                                           int64_t epool_elems, int64_t sink_elems, int nsink,
@@ -1319,11 +1322,19 @@ int kv800_hip_window_keys(const kv800_paged_t* P, int64_t R, int64_t max_rows, c
   KV800_REQUIRE(P->ebs > 0 && P->win > 0, "window_keys: ebs and win must be > 0");
   KV800_REQUIRE(((uintptr_t)k_out % 16) == 0 && ((uintptr_t)v_out % 16) == 0,
                 "window_keys: outputs must be 16-byte aligned");
-  KV800_REQUIRE(R <= 65535 && max_rows < (1ll << 31), "window_keys: at most 65535 rows of 2^31 keys per call");
-  hipLaunchKernelGGL(window_keys_kernel, dim3((unsigned)((max_rows + WIN_ROWS - 1) / WIN_ROWS), (unsigned)R), dim3(256), 0,
-                     (hipStream_t)stream, *P, cos_t, sin_t, rope_rows, epool_elems, sink_elems, (int)nsink, prev, ksl,
-                     qsl, k, v, k_out, v_out, kp);
-  return check_launch("window_keys");
+  KV800_REQUIRE(max_rows < (1ll << 31), "window_keys: rows of 2^31 keys and more");
+  for (int64_t r0 = 0; r0 < R; r0 += MAX_GRID_Y) {   // one launch, but for more rows than a grid's y holds
+    kv800_paged_t rows = *P;
+    rows.eoff += r0 * P->eoff_stride;
+    if (nsink) { rows.skoff += r0; rows.svoff += r0; }
+    hipLaunchKernelGGL(window_keys_kernel,
+                       dim3((unsigned)((max_rows + WIN_ROWS - 1) / WIN_ROWS), (unsigned)std::min(R - r0, MAX_GRID_Y)),
+                       dim3(256), 0, (hipStream_t)stream, rows, cos_t, sin_t, rope_rows, epool_elems, sink_elems,
+                       (int)nsink, prev + r0, ksl + r0, qsl + r0, k, v, k_out, v_out, kp);
+    const int rc = check_launch("window_keys");
+    if (rc != KV800_OK) return rc;
+  }
+  return KV800_OK;
 }
 
 }  // extern "C"

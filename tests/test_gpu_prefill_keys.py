@@ -87,3 +87,30 @@ def test_prefill_keys_new_rows(hip):
         assert same(K[s:s + prev[r]], hk[o:o + prev[r]]) and same(V[s:s + prev[r]], hv[o:o + prev[r]]), r
         assert same(K[s + prev[r]:rows.ksl[r + 1]], rotate(k[a:b], at, cos, sin)), r
         assert same(V[s + prev[r]:rows.ksl[r + 1]], v[a:b]), r
+
+
+def test_window_keys_many_rows(hip):
+    """More rows than the y extent of one grid."""
+    import lfm3_kv800_amd.kv800 as kv
+    R, ebs = 65535 + 5, 4
+    g = torch.Generator(device=DEV).manual_seed(9)
+    bf = lambda *s: torch.randn(*s, generator=g, device=DEV).to(torch.bfloat16)
+    prev = [r % 3 for r in range(R)]
+    ev, page = bf(7, 4, ebs, 256), torch.randint(0, 7, (R, 1), generator=g, device=DEV)
+    sk, sv, so = bf(3, 4, 4, 128), bf(3, 4, 4, 128), torch.randint(0, 3, (R,), generator=g, device=DEV)
+    k, v, cos, sin = bf(R, 4, 128), bf(R, 4, 128), bf(8, 32), bf(8, 32)
+    P = kv.Paged(epool=ev, eoff=page * ev.stride(0), ebs=ebs, e_hs=ev.stride(1), e_ts=ev.stride(2), e_v=128, sk=sk, sv=sv,
+                 skoff=so * 2048, svoff=so * 2048)
+    rows = rows_of(prev, [1] * R, hip.window_counts(prev, 2, 4))   # the last position, and position 0 as a sink before it
+    print("window_keys", R, flush=True)
+    K, V, kp = hip.window_keys(P, rows, k, v, cos, sin, 2, 4)
+    p = torch.tensor(prev, device=DEV)
+    at = torch.tensor(rows.ksl, device=DEV)
+    new, old, sink = at[1:] - 1, at[1:][p > 0] - 2, at[:-1][p > 1]
+    want_k, want_v = torch.empty_like(K), torch.empty_like(V)
+    pos = torch.zeros(len(K), dtype=torch.int64, device=DEV)
+    want_k[new], want_v[new], pos[new] = k, v, p
+    last = ev[page[p > 0, 0], :, p[p > 0] - 1]
+    want_k[old], want_v[old], pos[old] = last[..., :128], last[..., 128:], p[p > 0] - 1
+    want_k[sink], want_v[sink] = sk[so[p > 1], 0], sv[so[p > 1], 0]
+    assert torch.equal(kp.long(), pos) and same(V, want_v) and same(K, rotate(want_k, pos, cos, sin))
