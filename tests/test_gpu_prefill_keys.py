@@ -114,3 +114,32 @@ def test_window_keys_many_rows(hip):
     want_k[old], want_v[old], pos[old] = last[..., :128], last[..., 128:], p[p > 0] - 1
     want_k[sink], want_v[sink] = sk[so[p > 1], 0], sv[so[p > 1], 0]
     assert torch.equal(kp.long(), pos) and same(V, want_v) and same(K, rotate(want_k, pos, cos, sin))
+
+
+@pytest.mark.parametrize("rot", [True, False])
+def test_history_negative_key_scales(hip, oracle, rot):
+    """Sub-blocks written by hand with negative K scales and a lo of -0, which the quantizer never writes: a zero code times
+    such a scale is -0, whose sign the rotation of the dims without a frequency (cos 1, sin 0) can change."""
+    import numpy as np
+    import lfm3_kv800_amd.kv800 as kv
+    rng = np.random.default_rng(8)
+    sb = rng.integers(0, 256, (2, 51200), dtype=np.uint8)
+    scale = rng.choice(np.arange(0x20, 0x50, dtype=np.uint8), (2, 2048)).reshape(2, -1)
+    scale[:, 512:1024] &= 0x7F                       # V scales
+    scale[:, 1024:1536] = np.where(rng.random((2, 512)) < 0.5, 0x80, scale[:, 1024:1536])        # lo -0
+    scale[:, 1536:] |= np.where(rng.random((2, 512)) < 0.5, np.uint8(0x80), np.uint8(0))
+    sb[:, 49152:] = scale
+    kb, vf = oracle.dequantize_blocks(sb)
+    k = torch.from_numpy(kb.reshape(-1, 4, 128).view(np.int16)).view(torch.bfloat16).to(DEV)
+    assert ((k == 0) & torch.signbit(k)).any()
+    want_v = torch.from_numpy(vf.reshape(-1, 4, 128)).to(DEV).to(torch.bfloat16)
+    g = torch.Generator(device=DEV).manual_seed(8)
+    cos, sin = (torch.randn(512, 32, generator=g, device=DEV).to(torch.bfloat16) for _ in range(2))
+    at = torch.arange(512, device=DEV)
+    ev = torch.zeros(1, 4, 64, 256, dtype=torch.bfloat16, device=DEV)
+    P = kv.Paged(qpool=torch.from_numpy(sb).to(DEV), boff=torch.tensor([[0, 51200]], device=DEV), epool=ev,
+                 eoff=torch.zeros(1, 8, dtype=torch.int64, device=DEV), ebs=64, e_hs=ev.stride(1), e_ts=ev.stride(2), e_v=128,
+                 NQ=torch.tensor([2], dtype=torch.int32, device=DEV))
+    print("history negative scales", rot, flush=True)
+    K, V, _ = hip.history(P, [512], *((cos, sin) if rot else ()))
+    assert same(V, want_v) and same(K, rotate(k, at, cos, sin) if rot else k)
