@@ -375,15 +375,6 @@ def launch_flushes(layers, metas, mq, max_new=1):
 
 
 # ---------------------------------------------------------------- prefill / extend rows over compressed history
-def _ranges(starts, counts):
-    """Concatenation of range(s, s + c) over the pairs, as an int64 numpy array."""
-    starts, counts = np.asarray(starts, np.int64), np.asarray(counts, np.int64)
-    if counts.sum() == 0:
-        return np.zeros(0, np.int64)
-    base = np.repeat(starts - np.concatenate(([0], np.cumsum(counts)[:-1])), counts)
-    return base + np.arange(int(counts.sum()), dtype=np.int64)
-
-
 def _rows(qsl, counts, prev, dev):
     """PrefillRows of rows with `counts` keys before their new rows qsl[i] .. qsl[i + 1], from position prev[i] on."""
     if any(n < 0 for n in prev):

@@ -78,15 +78,6 @@ def test_plan_rules():
     assert spb == 32 and ns == 4
 
 
-def test_ranges_helper():
-    """vllm_cache._ranges: the concatenated key / position ranges the prefill rows assemble on the host."""
-    from lfm3_kv800_amd import vllm_cache as vc
-    got = vc._ranges([5, 0, 100, 7], [3, 0, 2, 1])
-    assert got.tolist() == [5, 6, 7, 100, 101, 7]
-    assert vc._ranges([], []).tolist() == []
-    assert vc._ranges([3], [0]).tolist() == []
-
-
 def test_host_to_device_on_cpu():
     """kv800_hip.host_to_device: lists, numpy arrays and tensors become tensors of the asked dtype on the device (on
     the CPU here; on a GPU the copy goes through pinned memory, asynchronously)."""
