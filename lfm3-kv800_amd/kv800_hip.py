@@ -135,10 +135,6 @@ def _stream(dev):
     return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
 
 
-def _stream_key(dev):
-    return torch.cuda.current_stream(dev).cuda_stream if dev.type == "cuda" else 0
-
-
 def _extent(t):
     """Elements from t's first element to the end of its storage (what the kernels may address from data_ptr)."""
     return t.untyped_storage().nbytes() // t.element_size() - t.storage_offset()
@@ -404,8 +400,7 @@ class PrefillRows:
 
     def __init__(self, qsl, ksl, qpos0, dev):
         qsl, ksl, qpos0 = [int(x) for x in qsl], [int(x) for x in ksl], [int(x) for x in qpos0]
-        dev = torch.device(dev)
-        if dev.type == "cuda" and dev.index is None:
+        if dev.index is None and dev.type == "cuda":
             dev = torch.device("cuda", torch.cuda.current_device())
         R = self.R = len(qpos0)
         if len(qsl) != R + 1 or len(ksl) != R + 1:
@@ -431,13 +426,12 @@ class PrefillRows:
         if any(s[r + 1] - s[r] != c + q[r + 1] - q[r] for r, c in enumerate(counts)):
             raise ValueError("ksl does not match the rows' history and new rows")
 
-    def ptrs(self):
-        """Device pointers of (qsl, ksl, qpos0, tiles) for launches on the current stream; the tensor behind them lives as
-        long as this object. One upload per stream: another stream would neither wait for it nor keep its memory."""
-        key = _stream_key(self.dev)
-        meta = self._meta.get(key)
+    def ptrs(self, stream):
+        """Device pointers of (qsl, ksl, qpos0, tiles) for launches on the current stream, `stream`; the tensor behind them
+        lives as long as this object. One upload per stream: another would neither wait for it nor keep its memory."""
+        meta = self._meta.get(stream.value)
         if meta is None:   # of two threads on one stream both take the first's
-            meta = self._meta.setdefault(key, host_to_device(self._host, torch.int64, self.dev))
+            meta = self._meta.setdefault(stream.value, host_to_device(self._host, torch.int64, self.dev))
         p, n = meta.data_ptr(), self.R + 1
         return tuple(ctypes.c_void_p(p + 8 * i) for i in (0, n, 2 * n, 3 * n - 1))
 
@@ -478,10 +472,11 @@ def prefill_rows(q, rows, K, V, kp, window=0, nsink=0, splits=None):
     splits = int(splits)
     T = qsl[-1]
     part = torch.empty(T * 16 * splits * 132 if splits > 1 else 0, dtype=torch.float32, device=dev)
-    m_qsl, m_ksl, m_pos, m_tiles = rows.ptrs()
+    stream = _stream(dev)
+    m_qsl, m_ksl, m_pos, m_tiles = rows.ptrs(stream)
     _check(L.kv800_hip_prefill_split(_ptr(q), m_qsl, m_pos, _ptr(K), _ptr(V), _ptr(kp), m_ksl, m_tiles, R, rows.ntiles, T,
                                      int(window), int(nsink), splits, _ptr(part) if splits > 1 else None, part.numel(),
-                                     _ptr(out), _stream(dev)))
+                                     _ptr(out), stream))
     return out
 
 
@@ -550,10 +545,11 @@ def prefill_keys(P, rows, k, v, cos_t, sin_t):
         s, qbytes, eelems = Paged(), 0, 0
         s.epool = s.eoff = s.NQ = K.data_ptr()
         s.ebs = 1
-    m_qsl, m_ksl, m_pos, _ = rows.ptrs()
+    stream = _stream(dev)
+    m_qsl, m_ksl, m_pos, _ = rows.ptrs(stream)
     _check(L.kv800_hip_prefill_keys(ctypes.byref(s), R, max(prev), max(b - a for a, b in zip(rows.qsl, rows.qsl[1:])),
                                     _ptr(cos_t), _ptr(sin_t), cos_t.shape[0], qbytes, eelems, m_pos, m_qsl, m_ksl,
-                                    _ptr(k), _ptr(v), _ptr(K), _ptr(V), _stream(dev)))
+                                    _ptr(k), _ptr(v), _ptr(K), _ptr(V), stream))
     return K, V
 
 
@@ -596,12 +592,13 @@ def window_keys(P, rows, k, v, cos_t, sin_t, win, nsink):
             raise IndexError("skoff / svoff must cover the rows")
         s.sk, s.sv, s.skoff, s.svoff = P.sk.data_ptr(), P.sv.data_ptr(), skoff.data_ptr(), svoff.data_ptr()
         sink_elems = min(_extent(P.sk), _extent(P.sv))
-    m_qsl, m_ksl, m_pos, _ = rows.ptrs()
+    stream = _stream(dev)
+    m_qsl, m_ksl, m_pos, _ = rows.ptrs(stream)
     rot = cos_t is not None
     _check(L.kv800_hip_window_keys(ctypes.byref(s), R, max(b - a for a, b in zip(rows.ksl, rows.ksl[1:])),
                                    _ptr(cos_t) if rot else None, _ptr(sin_t) if rot else None,
                                    cos_t.shape[0] if rot else 0, _extent(P.epool), sink_elems, nsink, m_pos, m_qsl, m_ksl,
-                                   _ptr(k), _ptr(v), _ptr(K), _ptr(V), _ptr(kp), _stream(dev)))
+                                   _ptr(k), _ptr(v), _ptr(K), _ptr(V), _ptr(kp), stream))
     return K, V, kp
 
 

@@ -1,5 +1,7 @@
 """Row geometry of prefill calls on the host: what the key assembly's launches would read or write out of range is
 refused before any launch, as the gathers refused it."""
+from ctypes import c_void_p
+
 import pytest
 import torch
 
@@ -52,7 +54,7 @@ def test_calls_refuse_queries_of_another_device(monkeypatch, call):
     import lfm3_kv800_amd.kv800 as kv
     lib = Calls()
     monkeypatch.setattr(kv800_hip, "ops", lambda: lib)
-    monkeypatch.setattr(kv800_hip, "_stream", lambda dev: None)
+    monkeypatch.setattr(kv800_hip, "_stream", lambda dev: c_void_p(0))
     bf = dict(dtype=torch.bfloat16)
     P = kv.Paged(epool=torch.zeros(1, 4, 64, 256, **bf), eoff=torch.zeros(1, 1, dtype=torch.int64), ebs=64, e_hs=64 * 256,
                  e_ts=256, e_v=128, NQ=torch.zeros(1, dtype=torch.int32))
@@ -64,15 +66,9 @@ def test_calls_refuse_queries_of_another_device(monkeypatch, call):
     assert len(lib.made) == 2   # the assembly and the attention
 
 
-def test_one_upload_per_stream(monkeypatch):
+def test_one_upload_per_stream():
     from lfm3_kv800_amd import kv800_hip
-    stream = [1]
-    monkeypatch.setattr(kv800_hip, "_stream_key", lambda dev: stream[0], raising=False)
     rows = kv800_hip.PrefillRows([0, 5], [0, 12], [7], CPU)
-    at = lambda: [p.value for p in rows.ptrs()]
-    first = at()
-    stream[0] = 2
-    second = at()
-    assert set(first).isdisjoint(second) and at() == second
-    stream[0] = 1
-    assert at() == first
+    at = lambda stream: [p.value for p in rows.ptrs(c_void_p(stream))]
+    first, second = at(0), at(64)
+    assert set(first).isdisjoint(second) and at(64) == second and at(0) == first
