@@ -1,4 +1,4 @@
-"""Benchmark of the 800h decode path on one MI355X, config C3 of BASELINE.json: one layer of paged split-K decode attention
+"""Benchmark of the 800h decode path on one MI355X: one layer of paged split-K decode attention
 over 64 sequences x 32,768 tokens (127 quantized 256-token sub-blocks + 256 exact tokens per sequence, permuted page
 tables), 16 query heads over 4 KV heads x 128 (the reference format's head shape; same bytes and flops per token as
 32 / 8 / 64).
@@ -18,8 +18,8 @@ launch duration, K launches back to back between one HIP event pair on their own
 committed rocprofv3 counter summary;
 cpu_baseline: a pure-torch CPU restatement of the reference's torch_decode.py on a sample of the same rows (the C
 oracle's time beside it). Extra
-fields: flush_c2 (config C2, the flush kernel alone), c4 (config 4, one decode step of all 6 attention
-layers over 398 ragged sequences), e2e (config 5, greedy decode tok/s of an LFM3-shaped model over 256
+fields: flush_c2 (C2, the flush kernel alone), c4 (C4, one decode step of all 6 attention
+layers over 398 ragged sequences), e2e (C5, greedy decode tok/s of an LFM3-shaped model over 256
 sequences), e2e_398x32k (the same loop at the reference's published point, 398 sequences of 32K tokens), prefill
 (prefill over compressed history: 8 rows x a 2048-token chunk over 16K-token histories, the attention kernel against
 the MFMA peak), fake_quant (training fake quantization of one layer's K and V), window_398 (one window + sinks layer
@@ -132,14 +132,10 @@ C2_B, C2_N, C2_EBS = 64, 2048, 128
 C2_NQ = (C2_N - 128) // 256                         # 7 flushed sub-blocks per sequence (kv800.py:433 flush rule)
 C2_READ = C2_B * C2_NQ * 256 * 4 * 128 * 2 * 2      # bf16 K + V gathered from the exact pages
 C2_WRITE = C2_B * C2_NQ * 51200
-C2_FMA = C2_B * C2_NQ * 256 * 4 * 16 * 688          # fp32 fma of the V Hadamard as sequential chains with shared
-                                                    # prefixes, 86 per output: a measure of the work, of which the
-                                                    # kernel forms most on the matrix cores (fma_frac may exceed 1)
-FMA_PEAK = 256 * 64 * 2.4e9                         # non-packed fp32 fma/s: 256 CUs x 64 lanes x 2.4 GHz
 
 
 def bench_flush_c2(torch, kh, dev, steps, warmup):
-    """config C2, the flush kernel alone: 64 sequences x a 2048-token prefill chunk in vLLM-geometry exact
+    """C2, the flush kernel alone: 64 sequences x a 2048-token prefill chunk in vLLM-geometry exact
     pages (128 tokens x 4 heads x [K128 | V128] bf16 per page, shuffled physical pages), K / V ~ N(0,1) with 1 % of
     the elements x 8, flushed by one launch into shuffled 1280-token quant pages (5 x 51,200 B per 262,144-B page):
     448 sub-blocks. Per-launch HIP events on the current stream."""
@@ -176,8 +172,7 @@ def bench_flush_c2(torch, kh, dev, steps, warmup):
     return {"workload": "C2: flush of 64 seqs x 2048-token chunk = 448 sub-blocks, vLLM page geometry, shuffled "
                         "exact and quant page tables, N(0,1) K/V with 1% outliers x8",
             "ms": round(ms, 5), "bytes": C2_READ + C2_WRITE, "gbps": round(gbps, 1),
-            "hbm_frac": round(gbps / HBM_PEAK_GBS, 4), "bound": "valu",
-            "fma_per_launch": C2_FMA, "fma_frac": round(C2_FMA / (ms * 1e-3) / FMA_PEAK, 4)}
+            "hbm_frac": round(gbps / HBM_PEAK_GBS, 4)}
 
 
 C4_R, C4_MIN, C4_MAX = 398, 1024, 32768
@@ -185,7 +180,7 @@ C4_GROUP = {6: "A", 14: "A", 22: "A", 2: "B", 10: "B", 18: "B"}   # two exact KV
 
 
 def bench_c4(torch, kh, dev, steps, warmup, cos, sin):
-    """config C4: the 6 attention layers of an LFM3-1.7B-shaped stack (quantized 6, 10, 14, 22; window + sinks
+    """C4: the 6 attention layers of an LFM3-1.7B-shaped stack (quantized 6, 10, 14, 22; window + sinks
     2, 18) over 398 sequences with lengths U[1K, 32K] (seeded), vLLM page geometry (exact: 128-token pages in two exact
     KV groups; quant: 1280-token pages in one group, sinks in the hosts' aux), one decode step per layer per step:
     the new token's rows, the flush of the sub-blocks that became eligible, decode tables and decode
@@ -266,7 +261,7 @@ E2E_R, E2E_MIN, E2E_MAX = 256, 1024, 32768
 
 
 def bench_e2e(torch, dev, steps, lens=None, seed=51, graph=False):
-    """config C5: greedy decode of a random-init LFM3-1.7B-shaped model (lfm3-kv800_amd/model.py: 24 layers,
+    """C5: greedy decode of a random-init LFM3-1.7B-shaped model (lfm3-kv800_amd/model.py: 24 layers,
     13 short-conv, 6 full-attention on the 800h caches, 5 sliding-window; weights N(0, 0.02) bf16) over 256 sequences
     with prompt lengths U[1K, 32K] (seeded), `steps` greedy steps; `lens` replaces the prompt lengths (the reference's
     published throughput point is 398 sequences of 32,768 tokens, RESULTS_RELEASE.md:90-96). tok/s = c (steps - 1) /
@@ -416,7 +411,8 @@ def bench_prefill(torch, kh, dev, steps, warmup):
             "ms": round(ms, 4), "tok_s": round(T / (ms * 1e-3), 1), "attention_kernel_ms": round(ms_k, 4),
             "attention_flop": flop, "tflops": round(tflops, 1), "mfma_frac": round(tflops / MFMA_BF16_PEAK, 4),
             "bound": "mfma",
-            "short_chunk_us": {"workload": f"1 row x 16 queries over a {PF_HIST}-token history (key-split path)",
+            "short_chunk_us": {"workload": f"1 row x 16 queries over a {PF_HIST}-token history (key-split path), one call "
+                                           "at a time with its host preparation",
                                "attention_call_us": short}}
 
 
@@ -603,7 +599,7 @@ C1_B, C1_N, C1_ITERS = 4, 1024, 10
 
 
 def build_c1(torch, dev):
-    """config C1: one quantized layer of 4 sequences x 1024 tokens in PagedStore's default geometry
+    """C1: one quantized layer of 4 sequences x 1024 tokens in PagedStore's default geometry
     (ebs 64, ring of 10 pages), q / K / V ~ N(0, 1) bf16 from seed 1, written and flushed by this build's HIP path
     (3 sub-blocks + 256 exact tokens per row). Returns (Paged, q, cos, sin) on the device."""
     import lfm3_kv800_amd.kv800 as kv
@@ -796,7 +792,7 @@ def main():
                    C(q1), C(cos1), C(sin1))
         del P1, q1, cos1, sin1
 
-    # ---- the other BASELINE.json configs with a GPU workload: C2 (flush alone), C4 (6-layer decode step), C5 (engine loop)
+    # ---- the other workloads with a GPU workload: C2 (flush alone), C4 (6-layer decode step), C5 (engine loop)
     del layers, structs
     torch.cuda.empty_cache()
     extra_steps = max(5, min(a.steps, 20))

@@ -1,13 +1,13 @@
 """Pure-torch CPU restatement of the reference's torch decode path -- TEST INFRASTRUCTURE, not product code.
 
-bench.py times it on the GPU box's host cores as the CPU baseline (`cpu_baseline.kind = "port"`): the reference's own
+bench.py times it on the host cores as the CPU baseline (`cpu_baseline.kind = "port"`): the reference's own
 pure-torch backend (lfm3_kv800/torch_decode.py:27-80, with the dequantizer of kv800.py:79-92) cannot travel to the
 box, so this file states the same algorithm on CPU torch -- per row, the flushed sub-blocks dequantized (2-bit K codes
 times the fp8 scale plus the fp8 offset, rounded to bf16; 1-bit V planes times the scale plus the offset, times the
 normalised Hadamard), the exact rows gathered from their pages, the sinks of window layers, every key rotated on the
 dim pairs (d, d + 64), d < 32, in fp32 and rounded to bf16, then one fp32 softmax over all positions (scale 128^-0.5)
 with 4 query heads per KV head. tests/test_oracle.py pins it against the C oracle (oracle/kv800_oracle.c) on the
-config C1 inputs. Only tests/ and bench.py's cpu_baseline leg import it."""
+C1 inputs. Only tests/ and bench.py's cpu_baseline leg import it."""
 import torch
 
 BLK, SUB, NSINK = 256, 51200, 4

@@ -1,4 +1,4 @@
-"""The LFM3-shaped decode model (lfm3-kv800_amd/model.py, config C5) on an MI355X: its attention layers on the
+"""The LFM3-shaped decode model (lfm3-kv800_amd/model.py, C5) on an MI355X: its attention layers on the
 HIP path (vLLM page geometry: quantized, window + sinks and native sliding layers) against the same model, same
 weights and conv states, whose attention is the CPU oracle's torch_decode restatement over each layer's full K / V
 history (quantized by the oracle quantizer, sinks and windows as torch_decode.py:27-80 selects them). Teacher forcing:
@@ -235,7 +235,7 @@ def _decode_setup(lens0, steps):
 
 
 def test_model_full_size_c5(hip, oracle):
-    """config C5 at full size: 256 rows with prompt lengths U[1K, 32K] (the bench's seed), the
+    """C5 at full size: 256 rows with prompt lengths U[1K, 32K] (the bench's seed), the
     prompt caches written through the attention layers' step path in 2048-token prefill chunks
     (PagedAttention800.fill -> vllm_cache write_step: exact pages, sinks, flushes), then 3 greedy steps of the
     LFM3-shaped model: every step's logits finite and tokens in range; sub-blocks the fill flushed (first, middle and

@@ -164,7 +164,7 @@ def test_flush_two_kv_groups(hip, oracle, latency):
 
 
 def test_flush_c2_full_size(hip, oracle):
-    """config C2 at full size: 64 sequences x a 2048-token chunk in vLLM-geometry exact pages (shuffled), K / V
+    """C2 at full size: 64 sequences x a 2048-token chunk in vLLM-geometry exact pages (shuffled), K / V
     ~ N(0,1) with 1 % of the elements x 8, one flush launch into shuffled 1280-token quant pages: all 448 sub-blocks
     (the flush rule gives 7 per sequence) must equal the oracle quantizer's bytes."""
     B, n, ebs = 64, 2048, 128
@@ -245,7 +245,7 @@ def test_decode_reference_cases(hip, oracle, win, n, seed):
 
 @pytest.mark.parametrize("B,n", [(4, 1024), (2, 384), (3, 5000), (1, 9000)])
 def test_decode_baseline_inputs(hip, oracle, B, n):
-    """config C1 (B = 4, n = 1024, q / K / V ~ N(0, 1)) and other lengths, shuffled pages: the strict bar."""
+    """C1 (B = 4, n = 1024, q / K / V ~ N(0, 1)) and other lengths, shuffled pages: the strict bar."""
     rng = np.random.RandomState(B * 1000 + n)
     K = oracle.randn_bf16(rng, (B, n, 4, 128)); V = oracle.randn_bf16(rng, (B, n, 4, 128))
     q = oracle.randn_bf16(rng, (B, 16, 128))
@@ -406,7 +406,7 @@ def test_decode_merge_many_partials(hip, oracle):
 
 
 def test_decode_full_size_all_rows(hip, oracle):
-    """config C3 at full size (64 x 32,768, permuted tables): cache built on the GPU by the HIP quantizer,
+    """C3 at full size (64 x 32,768, permuted tables): cache built on the GPU by the HIP quantizer,
     decoded by the HIP kernels; every row is decoded again by the oracle from the downloaded pages (the strict bar), and
     every output is finite and within the range of its row's dequantized values."""
     import lfm3_kv800_amd.kv800 as kv

@@ -184,7 +184,7 @@ def test_step_meta_matches_torch(hip):
 
 
 def test_vllm_decode_step_full_size(hip, oracle):
-    """the shape of config C4 through the vLLM cache path, all six attention layers: 398 rows with
+    """the shape of C4 through the vLLM cache path, all six attention layers: 398 rows with
     lengths U[1K, 32K] (rows 0-7 placed so the step flushes a sub-block), window + sinks layers 2 and 18 (sinks in the
     aux areas of 6 / 10 and 14 / 22) and quantized layers 6, 10, 14, 22, in two exact KV groups (A: 6, 14, 22; B: 2,
     10, 18). Each row's history is a slice of a per-layer N(0,1) pool; its last 640 positions sit in a ring of 8
