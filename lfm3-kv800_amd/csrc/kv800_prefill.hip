@@ -30,15 +30,17 @@
 // tile whose keys are all in range, precede the workgroup's first query and lie in its last query's window (or are sinks)
 // is not masked.
 // Bound: matrix and VALU issue, which overlap only in part, at the clock the part holds under them (1.9 GHz here). 32 x 32
-// MFMA instead of twice as many 16 x 16 ones, with half the cross-lane steps, and the phase priorities: 8 rows x 2048
-// queries over 16K keys, whole call, 2,424 -> 2,370 -> 2,240 us (this kernel about 1.03 PFLOP/s; a library product of
-// 8192^3 reaches 1.14 on the same card).
+// MFMA instead of twice as many 16 x 16 ones, with half the cross-lane steps, and the phase priorities: 8 ragged rows of up
+// to 2048 queries over up to 16K keys (2.2 TFLOP), whole call, 2,424 -> 2,370 -> 2,240 us on one box, 2,120-2,200 us on
+// others (this kernel 1.03-1.07 PFLOP/s; a library product of 8192^3 reaches 1.14 on the same card). MFMA busy 58 % of the
+// SIMD cycles, waves wait in 61 % of theirs at 1.85 per SIMD; the LDS counts two conflict cycles per MFMA, which the 16 x 16
+// reads did not have, and waves wait for it in 4 %.
 // Key tiles outside [first key a query of the workgroup can see, last key not in its future] are skipped: for window
 // layers only the sink keys and the keys of the window are read, as one list (template flag WIN: its addresses cost the
 // windowless kernel 4 %). A window workgroup has 5 tiles, so its start counts as much: the row and the three key bounds
-// are found by 64-way searches side by side, behind the query loads. 8 rows x 2048 queries, window 256 + 4 sinks, whole call: 131 us
-// with a sink tile, masks on every tile and one search after the other, 117 us now (34 GFLOP, 134 MB of Q and output:
-// latency of the tiles' loads, two workgroups per CU).
+// are found by 64-way searches side by side, behind the query loads. 8 rows x 2048 queries, window 256 + 4 sinks, whole
+// call: 131 us with a sink tile, masks on every tile and one search after the other, 117 us now (34 GFLOP, 134 MB of Q and
+// output: latency of the tiles' loads, two workgroups per CU).
 // The grid is one workgroup per (KV head, 32-query tile), numbered so that each XCD runs whole (KV head, row) runs of
 // tiles: the 64 workgroups of a 2048-query chunk walk the same key tiles together through one L2.
 #include "kv800_common.h"
@@ -94,8 +96,8 @@ __device__ __forceinline__ uint32_t bfpk(float a, float b) {
 // and the workgroups of one (KV head, row) run on one XCD, in order, so the row's key tiles are read once into that
 // XCD's L2 for its 64 query tiles. Keys come in tiles of 64, loaded into LDS as K and V rows by LDS-direct loads (no
 // register staging) and double-buffered: the next tile's loads are in flight while the current one is multiplied, one
-// barrier per tile. A tile that every query of the workgroup sees whole needs no mask: in a chunk over a long history, nearly
-// every tile.
+// barrier per tile. A tile that every query of the workgroup sees whole needs no mask: in a chunk over a long history,
+// nearly every tile.
 constexpr int PQ = 32;      // queries per workgroup = per interface tile (tile_off counts these)
 constexpr int PPART = 132;  // floats per key-split partial of (query, head): 128 dims of o, m, l, 2 of padding
 constexpr int PMAXSPLIT = 256;
@@ -373,7 +375,8 @@ prefill_kernel(const uint16_t* __restrict__ q, const int64_t* __restrict__ qsl, 
     for (int j = 0; j < 4; ++j)
 #pragma unroll
       for (int c = 0; c < 4; ++c)
-        *reinterpret_cast<f4*>(pp + 32 * j + 8 * c + 4 * G) = f4{o[j][4 * c], o[j][4 * c + 1], o[j][4 * c + 2], o[j][4 * c + 3]};
+        *reinterpret_cast<f4*>(pp + 32 * j + 8 * c + 4 * G) =
+            f4{o[j][4 * c], o[j][4 * c + 1], o[j][4 * c + 2], o[j][4 * c + 3]};
     if (G == 0) { pp[128] = m; pp[129] = l; }
     return;
   }
@@ -394,8 +397,9 @@ prefill_kernel(const uint16_t* __restrict__ q, const int64_t* __restrict__ qsl, 
 // loads in flight during the reductions, the waves' sums added through LDS; out = bf16(O / L) (a split without keys has
 // l = 0 and o = 0). Bound: latency, of the partials other XCDs wrote. 4 waves per pair where one would leave most CUs
 // without a workgroup (up to 64 queries) and each of the 4 has several partials: whole attention call, 16 queries x 16K
-// keys in 64 splits 22.0 -> 16.9 us, 32 queries 24.9 -> 20.4, 64 queries x 4K keys in 32 splits 21.8 -> 21.1; but 128 queries
-// x 4K in 8 splits 22.4 -> 26.3, 64 queries x 16K in 16 splits 30.9 -> 31.9, so these keep one wave.
+// keys in 64 splits 22.0 -> 16.9 us (calls back to back: the kernels; one call at a time the host takes 34-35 us either
+// way), 32 queries 24.9 -> 20.4, 64 queries x 4K keys in 32 splits 21.8 -> 21.1; but 128 queries x 4K in 8 splits 22.4 ->
+// 26.3, 64 queries x 16K in 16 splits 30.9 -> 31.9, so these keep one wave.
 constexpr int64_t MERGE_WIDE_PAIRS = 1024;
 constexpr int MERGE_WIDE_SPLITS = 17;
 __device__ __forceinline__ float wave_max(float x) {
@@ -504,15 +508,16 @@ int kv800_hip_prefill_split(const uint16_t* q, const int64_t* qsl, const int64_t
                   (long long)part_floats, (long long)(T * 16 * splits * PPART));
   }
   const float scale_log2 = 0.088388347648318440f * 1.4426950408889634f;   // 128^-0.5 * log2(e)
-  hipLaunchKernelGGL(window > 0 ? prefill_kernel<true> : prefill_kernel<false>, dim3((unsigned)(ntiles * 4 * splits)), dim3(256), 0, (hipStream_t)stream, q, qsl,
-                     qpos0, K, V, kp, ksl, tile_off, R, window, nsink, scale_log2, out, (int)splits,
-                     splits > 1 ? part : (float*)nullptr);
+  hipLaunchKernelGGL(window > 0 ? prefill_kernel<true> : prefill_kernel<false>, dim3((unsigned)(ntiles * 4 * splits)),
+                     dim3(256), 0, (hipStream_t)stream, q, qsl, qpos0, K, V, kp, ksl, tile_off, R, window, nsink,
+                     scale_log2, out, (int)splits, splits > 1 ? part : (float*)nullptr);
   int rc = check_launch("prefill");
   if (rc != KV800_OK || splits == 1 || T == 0) return rc;
   const int64_t pairs = T * 16;
   const bool wide = pairs <= MERGE_WIDE_PAIRS && splits >= MERGE_WIDE_SPLITS;
-  hipLaunchKernelGGL(wide ? prefill_merge_kernel<4> : prefill_merge_kernel<1>, dim3((unsigned)(wide ? pairs : (pairs + 3) / 4)),
-                     dim3(256), 0, (hipStream_t)stream, part, pairs, (int)splits, out);
+  hipLaunchKernelGGL(wide ? prefill_merge_kernel<4> : prefill_merge_kernel<1>,
+                     dim3((unsigned)(wide ? pairs : (pairs + 3) / 4)), dim3(256), 0, (hipStream_t)stream, part, pairs,
+                     (int)splits, out);
   return check_launch("prefill_merge");
 }
 

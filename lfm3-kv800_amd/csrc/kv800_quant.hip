@@ -42,7 +42,7 @@ int check_launch(const char* what) {
 
 namespace {
 
-constexpr int QTHREADS = 512;    // 8 waves per sub-block, 32 tokens each
+constexpr int QTHREADS = 512;    // a K workgroup: one head of a sub-block; a V workgroup: a token range of it
 constexpr int QWPS = 4;          // waves per SIMD the throughput kernels are built for (two workgroups per CU)
 constexpr int QW = QTHREADS / 64;
 
@@ -529,8 +529,8 @@ __device__ __forceinline__ bool quick_v4(const uint4 (&in)[4], const SignB& sb, 
 }
 
 // V bits and scales of tokens [t0, t0 + 4 VG QW) of one sub-block: wave w takes VG groups of four consecutive tokens.
-// Lane (g, m) loads dims 8 g + 32 q .. + 7 of row m (four 16-byte pieces, every group's requested up front), the bf16 MFMA's A operand as
-// they are; for the exact chain the pieces' elements change places with the other lane groups' so
+// Lane (g, m) loads dims 8 g + 32 q .. + 7 of row m (four 16-byte pieces, every group's requested up front), the bf16
+// MFMA's A operand as they are; for the exact chain the pieces' elements change places with the other lane groups' so
 // that the lane holds x[m][4 s + g].
 constexpr int VSPLIT = 4, VTOK = BLK / VSPLIT, VTPW = VTOK / QW;
 
@@ -576,10 +576,11 @@ __device__ void quantize_v(const Src& src, uint8_t* __restrict__ out, int t0) {
 
 // A quantize grid holds, per sub-block, VSPLIT V workgroups (V is independent per token) and 4 K workgroups (one per
 // head: all 256 tokens per channel, each row read once). All V workgroups come first: they are the long ones, and the K
-// workgroups fill in behind them (448 sub-blocks: 90 us, 98-118 us interleaved, 100 us with K first, before the chain's tiles were
-// indexed at compile time). V alone takes about 60 us, K alone 40 us, both mostly the latency of one-shot workgroups at
-// two per CU; 448 sub-blocks of paged rows took 147 us with a scalar fma chain per V lane and the code arithmetic per K
-// element, and take 84 us now (3.1 TB/s).
+// workgroups fill in behind them (448 sub-blocks: 90 us, 98-118 us interleaved, 100 us with K first, before the chain's
+// tiles were indexed at compile time). V alone takes about 60 us, K alone 40 us, both mostly the latency of one-shot
+// workgroups at two per CU: by the counters VALU and MFMA issue takes 56 % of the SIMD cycles (bf16 MFMA busy 21 %) at 2.7
+// waves per SIMD, which wait in 73 % of theirs. 448 sub-blocks of paged rows took 147 us with a scalar fma chain per V
+// lane and the code arithmetic per K element, and take 84 us now (3.1 TB/s).
 // 32-bit throughout (the host bounds the grid): scalar compares and selects.
 struct Part { int unit; bool kpass; int part; };
 __device__ __forceinline__ Part part_of(int units, int vsplit) {
@@ -704,7 +705,9 @@ __device__ __forceinline__ float ubyte(uint32_t c, int e) { return (float)((c >>
 // One workgroup per quarter of a sub-block and side (its K, its V), so that 448 sub-blocks fill the part and the V
 // chains' workgroups run beside the K workgroups' stores. K: a lane keeps its 8 channels' scales in registers and a
 // wave writes whole 1 KB token rows. 448 sub-blocks: 205 us as one workgroup per sub-block with per-element scale
-// reads and vector chains, 122 us now (3.1 TB/s).
+// reads and vector chains, 122 us now (3.1 TB/s). The chains are 5.05 G FMA, 67 us of fp32 MFMA at 75 T FMA/s (MFMA busy 64 %
+// of the SIMD cycles, VALU 22 %), the 378 MB 73 us at the rate of a large copy: the V workgroups' scalar dword stores and
+// the K workgroups behind them overlap the chains only in part.
 constexpr int DPARTS = 4, DTOK = BLK / DPARTS;
 __global__ void __launch_bounds__(256) dequant_kernel(const uint8_t* __restrict__ sb, int M, uint16_t* __restrict__ kout,
                                                       float* __restrict__ vout) {
@@ -847,7 +850,8 @@ __global__ void __launch_bounds__(256) fake_quant_k4_kernel(const float* __restr
 // quantize -> dequantize round trip. A wave takes four tokens at a time through both chains on fp32 MFMA; lane (g, m)
 // loads the float4s 4 (4 u + g) of row m, whose elements change places with the other lane groups'. Between the chains
 // the code bytes and the scales go from the result's lanes to the next operand's through the wave's 320 bytes of LDS.
-// 32,768 tokens: 67 us with vector chains, 59 us now; bound: 42 us of fp32 MFMA beside the scales and bits on the VALU.
+// 32,768 tokens: 67 us with vector chains, 54-57 us now; bound: 2.9 G FMA, 38 us of fp32 MFMA at 75 T FMA/s (busy 76 % of the
+// SIMD cycles), beside the scales and bits on the VALU.
 constexpr int FQV_GROUPS = 2;   // groups of four tokens per wave
 struct FqvLds { uint32_t vb[16][4]; float sc[4][4]; };   // row's code bytes; token's (lo, scale) per pair of heads
 __global__ void __launch_bounds__(256) fake_quant_v_kernel(const float* __restrict__ v, int64_t N,
@@ -905,7 +909,8 @@ __global__ void __launch_bounds__(256) fake_quant_v_kernel(const float* __restri
 // rope table) are written as zeros. One workgroup per (hpos-position tile, row): hpos = 32 (two MFMA groups of four
 // tokens per wave), or 16 when 32 gives fewer than 1,024 workgroups (a single row). hpos divides 256, so a tile never
 // straddles a sub-block; the outputs do not depend on it. 8 rows of 16K positions: 212 us with vector chains and
-// software rounding, 134 us now (64 or 16 positions: 137 / 144 us); one row 48 -> 24 us. Bound: 84 us of fp32 MFMA.
+// software rounding, 134 us now (64 or 16 positions: 137 / 144 us); one row 48 -> 24 us. Bound: 5.8 G FMA, 77 us of fp32 MFMA
+// at 75 T FMA/s (busy 57 % of the SIMD cycles), beside 293 MB of stores.
 __device__ __forceinline__ void rope8(float (&a)[8], float (&b)[8], const uint16_t* cs, const uint16_t* sn, bool rope) {
   // a = dims d0 .. d0 + 7, b = dims d0 + 64 .. d0 + 71; rope: d0 < 32 (cs / sn the tables' entries d0 ..), else the
   // unrotated dims, for which the table holds cos 1, sin 0

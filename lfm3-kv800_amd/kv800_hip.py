@@ -380,9 +380,9 @@ def prefill_splits(tiles, max_key_tiles):
     """Key splits of one prefill launch: 1 when its tiles x 4 workgroups nearly fill the GPU, else enough for about
     512 workgroups, or 256 when that many would have fewer than PREFILL_SPLIT_TILES key tiles each (two workgroups on a CU
     gain about 15 % per tile, against twice the partials), with at least two 64-key tiles per split and at most 64 splits.
-    512 / 256 workgroups, whole attention call in us: 64 queries x 16K keys 33 / 26, 128 x 4K 27.9 / 23.0, 128 x 16K
-    39.1 / 34.7, 256 x 4K 30.1 / 27.1, 512 x 1K 26.2 / 21.8; but 256 x 16K 51.8 / 53.1, 512 x 16K 82 / 101, 128 x 64K
-    86 / 94."""
+    512 / 256 workgroups, attention calls back to back, in us: 64 queries x 16K keys 29.8 / 26.8, 128 x 4K 24.6 / 22.9, 128 x
+    16K 36.1 / 35.6, 256 x 4K 28.5 / 27.3, 512 x 1K 26.2 / 21.8; but 256 x 16K 50.5 / 55.7, 512 x 16K 82 / 96, 128 x 64K
+    89 / 96."""
     w = 4 * tiles
     if w >= PREFILL_SPLIT_BELOW or max_key_tiles < 4:
         return 1
